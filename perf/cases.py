@@ -141,52 +141,121 @@ def _normal(generator, shape, scale=1.0):
 
 def _on_device(tensor, dtype, device):
     """A block-float tensor, or bf16 tiles, as a model's loading code makes them."""
-    if dtype == ttnn.bfloat16:
-        tensor = tensor.bfloat16()
+    tensor = tensor.bfloat16() if dtype == ttnn.bfloat16 else tensor
     return ttnn.from_torch(tensor, dtype=dtype, layout=ttnn.TILE_LAYOUT, device=device)
 
 
-def prepare(case, seed):
+def _inputs(case, seed):
+    """The values of one pass as plain tensors, from the seed alone: what a block-float tensor is made from in fp32, the rest in
+    the type the path takes."""
     generator = torch.Generator(device="cuda")
     generator.manual_seed(seed)
-    device = ttnn.open_device(torch.cuda.current_device())
-    kind, state = case["kind"], {"kind": case["kind"]}
-    dtype = _DTYPE[case["weights"]]
+    kind = case["kind"]
 
     def activations(*shape):
-        return _on_device(_normal(generator, shape), ttnn.bfloat16, device)
+        return _normal(generator, shape).bfloat16()
 
     def weights(*shape, scale=0.02):
-        return _on_device(_normal(generator, shape, scale), dtype, device)
+        return _normal(generator, shape, scale)
 
     if kind == "from_torch":
-        source = _normal(generator, (case["batch"], 1, case["k"], case["n"]), 0.02)
-        state["host"] = (source if case["source"] == "fp32" else source.bfloat16()).cpu()
-        state["dtype"], state["device"] = dtype, device
-    elif kind == "to_torch":
-        state["x"] = weights(case["batch"], 1, case["k"], case["n"], scale=1.0)
-    elif kind == "attention":
+        source = weights(case["batch"], 1, case["k"], case["n"])
+        return {"host": source if case["source"] == "fp32" else source.bfloat16()}
+    if kind == "to_torch":
+        return {"x": weights(case["batch"], 1, case["k"], case["n"], scale=1.0)}
+    if kind == "attention":
         b, m, d = case["batch"], case["m"], case["k"]
-        state["q"], state["k_t"] = activations(b, _HEADS, m, d), weights(b, _HEADS, d, m, scale=1.0)
-        probabilities = torch.softmax(_normal(generator, (b, _HEADS, m, m)), dim=-1)
-        state["p"], state["v"] = _on_device(probabilities, ttnn.bfloat16, device), weights(b, _HEADS, m, d, scale=1.0)
+        values = {"q": activations(b, _HEADS, m, d), "k_t": weights(b, _HEADS, d, m, scale=1.0)}
+        values["p"] = torch.softmax(_normal(generator, (b, _HEADS, m, m)), dim=-1).bfloat16()
+        values["v"] = weights(b, _HEADS, m, d, scale=1.0)
+        return values
+    b, m, k, n = case.get("batch", 1), case["m"], case["k"], case["n"]
+    values = {"x": activations(b, 1, m, k)}
+    if kind == "linear":
+        values["w"] = weights(1, 1, k, n)
+        if case["bias"]:
+            values["bias"] = _normal(generator, (1, 1, 1, n), 0.1).bfloat16()
+    elif kind == "bmm":
+        values["w"] = weights(b, 1, k, n)
+    elif kind == "ffn":
+        values["w1"], values["w2"] = weights(1, 1, k, n), weights(1, 1, n, k)
+        values["b1"], values["b2"] = (_normal(generator, (1, 1, 1, width), 0.1).bfloat16() for width in (n, k))
+    elif kind == "mlp":
+        values["w1"], values["w2"] = weights(1, 1, k, n), weights(1, 1, n, k)
     else:
-        b, m, k, n = case.get("batch", 1), case["m"], case["k"], case["n"]
-        state["x"] = activations(b, 1, m, k)
-        if kind == "linear":
-            state["w"] = weights(1, 1, k, n)
-            state["bias"] = _on_device(_normal(generator, (1, 1, 1, n), 0.1), ttnn.bfloat16, device) if case["bias"] else None
-            state["activation"] = None if case["activation"] == "none" else case["activation"]
-        elif kind == "bmm":
-            state["w"] = weights(b, 1, k, n)
-        elif kind == "ffn":
-            state["w1"], state["w2"] = weights(1, 1, k, n), weights(1, 1, n, k)
-            state["b1"], state["b2"] = (_on_device(_normal(generator, (1, 1, 1, width), 0.1), ttnn.bfloat16, device) for width in (n, k))
-        elif kind == "mlp":
-            state["w1"], state["w2"] = weights(1, 1, k, n), weights(1, 1, n, k)
-        else:
-            state["w1"], state["w3"], state["w2"] = weights(1, 1, k, n), weights(1, 1, k, n), weights(1, 1, n, k)
+        values["w1"], values["w3"], values["w2"] = weights(1, 1, k, n), weights(1, 1, k, n), weights(1, 1, n, k)
+    return values
+
+
+_WEIGHTS = ("k_t", "v", "w", "w1", "w2", "w3")
+
+
+def prepare(case, seed):
+    device = ttnn.open_device(torch.cuda.current_device())
+    dtype, kind = _DTYPE[case["weights"]], case["kind"]
+    values, state = _inputs(case, seed), {"kind": kind}
+    if kind == "from_torch":
+        state["host"], state["dtype"], state["device"] = values["host"].cpu(), dtype, device
+        return state
+    for name, value in values.items():
+        state[name] = _on_device(value, dtype if name in _WEIGHTS or kind == "to_torch" else ttnn.bfloat16, device)
+    if kind == "linear":
+        state.setdefault("bias", None)
+        state["activation"] = None if case["activation"] == "none" else case["activation"]
     return state
+
+
+def _whole_tiles(x):
+    return torch.nn.functional.pad(x, (0, -x.shape[-1] % 32, 0, -x.shape[-2] % 32))
+
+
+def _tiles(x):
+    """The elements in the order of 32 x 32 tiles of four 16 x 16 faces, flat."""
+    x = _whole_tiles(x)
+    h, w = x.shape[-2:]
+    return x.reshape(-1, h // 32, 2, 16, w // 32, 2, 16).permute(0, 1, 4, 2, 5, 3, 6).reshape(-1)
+
+
+def _stored(x, weights):
+    """What a tensor of this type holds of x, in 64 bits: for block floats 16 neighbours share the largest one's exponent, and a
+    mantissa of 7 or 3 bits is rounded half up."""
+    if weights == "bf16":
+        return x.bfloat16().double()
+    bits = 7 if weights == "bfp8_b" else 3
+    groups = _whole_tiles(x).double()
+    shape = groups.shape
+    groups = groups.reshape(-1, 16)
+    step = torch.exp2(torch.frexp(groups.abs().amax(dim=1, keepdim=True))[1].double() - bits)
+    codes = torch.clamp(torch.floor(groups.abs() / step + 0.5), max=2 ** bits - 1)
+    return (torch.sign(groups) * codes * step).reshape(shape)
+
+
+def exact(case, seed):
+    kind, weights = case["kind"], case["weights"]
+    if kind == "from_torch":
+        return None
+    values = _inputs(case, seed)
+    if kind == "to_torch":
+        return _stored(values["x"], weights)[..., :case["k"], :case["n"]].cpu()
+    values = {name: _stored(value, weights) if name in _WEIGHTS else value.double() for name, value in values.items()}
+    # activations are stored in whole tiles: the rows and columns that fill them up are zeros, and part of the outputs
+    values = {name: value if name.startswith("b") else _whole_tiles(value) for name, value in values.items()}
+    act = {"none": lambda t: t, "gelu": torch.nn.functional.gelu, "silu": torch.nn.functional.silu, "relu": torch.relu}
+    pad_bias = lambda t: torch.nn.functional.pad(t, (0, -t.shape[-1] % 32))
+    x = values.get("x")
+    if kind == "attention":
+        return _tiles(values["q"] @ values["k_t"]), _tiles(values["p"] @ values["v"])
+    if kind == "linear":
+        product = x @ values["w"]
+        return _tiles(act[case["activation"]](product + pad_bias(values["bias"]) if case["bias"] else product))
+    if kind == "bmm":
+        return _tiles(x @ values["w"])
+    if kind == "mlp":
+        return _tiles(act["gelu"](x @ values["w1"]) @ values["w2"])
+    if kind == "gated_mlp":
+        return _tiles((act["silu"](x @ values["w1"]) * (x @ values["w3"])) @ values["w2"])
+    hidden = act["gelu"](x @ values["w1"] + pad_bias(values["b1"]))
+    return _tiles(_stored(hidden.bfloat16(), "bfp8_b") @ values["w2"] + pad_bias(values["b2"]))
 
 
 def run(state):
