@@ -202,9 +202,10 @@ TTMI_API void ttmi_matmul_bfp_plan(uint32_t batch, uint32_t m, uint32_t k, uint3
  * tt_eager/tt_dnn/op_library/bmm/bmm_op.hpp:388-456):  C[b, m, n] = act(A[b, m, k] . B[(b | 0), k, n] + bias[n]).
  *   b        bf16 in TILE layout (4-face tiles of 2048 bytes, tile (kt, nt) of slice s at index (s*Kt + kt)*Nt + nt), k and n
  *            multiples of 32
- * Everything else as for ttmi_matmul_bfp.  Two launches: the weights are re-laid-out into the operand layout of the matrix
+ * Everything else as for ttmi_matmul_bfp.  One launch that reads the weights where they lie (attention's batched products,
+ * outputs of few blocks); for large outputs two: the weights are re-laid-out into the operand layout of the matrix
  * cores (workspace: 2 bytes per weight, ttmi_matmul_bf16_workspace_bytes(); NULL = a buffer of the library), then the
- * bf16 GEMM that ttmi_matmul_bfp uses from 512 rows on runs on them.  Not a tuned path: block-float weights are. */
+ * bf16 GEMM that ttmi_matmul_bfp uses from 512 rows on runs on them. */
 TTMI_API size_t ttmi_matmul_bf16_workspace_bytes(uint32_t b_batch, uint32_t k, uint32_t n);
 TTMI_API int ttmi_matmul_bf16(const void *a, int a_layout, const void *b, uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k,
                      uint32_t n, const void *bias, int activation, void *c, int c_layout, int c_dtype, void *workspace,

@@ -710,8 +710,7 @@ def test_every_kernel_packs_a_block_float_output_in_its_epilogue(oracle, out_fmt
 
 @pytest.mark.parametrize("batch,b_batch,m,k,n", [(1, 1, 32, 64, 64), (1, 1, 32, 4544, 256), (2, 2, 40, 160, 96), (3, 1, 300, 96, 288), (1, 1, 512, 256, 544)])
 def test_bf16_weights(batch, b_batch, m, k, n):
-    """Two bf16 operands (ttmi_matmul_bf16): weights in TILE layout, re-laid-out and multiplied by the bf16 GEMM of the
-    expanding path; against a float64 matmul of the same values with the bound of the block-float GEMMs; TILE and
+    """Two bf16 operands (ttmi_matmul_bf16): weights in TILE layout; against a float64 matmul of the same values with the bound of the block-float GEMMs; TILE and
     row-major activations give the same bits; bias and activation; block-float output."""
     a_bits = workloads.activations_bf16(m, k, seed=500, batch=batch)
     w_bits = workloads.f32_to_bf16_bits_rne(workloads.weights_f32(k, n, seed=501, batch=b_batch))
@@ -736,6 +735,41 @@ def test_bf16_weights(batch, b_batch, m, k, n):
     ws = torch.full((need,), 0x5A, dtype=torch.uint8, device="cuda")
     again = capi.matmul_bf16(a_dev, capi.ROW_MAJOR, w_tiles, batch, b_batch, m, k, n, workspace=ws)
     assert torch.equal(again.view(torch.int16), c16.view(torch.int16))
+
+
+@pytest.mark.parametrize("block", [64, 128])
+@pytest.mark.parametrize("batch,b_batch,m,k,n", [(1, 1, 1, 32, 32), (1, 1, 33, 64, 96), (2, 2, 127, 96, 160), (3, 1, 160, 128, 288), (17, 17, 64, 160, 64)])
+def test_bf16_weights_read_in_place(oracle, batch, b_batch, m, k, n, block, knobs):
+    """The kernel that reads bf16 weights where they lie, at the edges of its blocks (rows, columns, fewer steps than stages of
+    its ring), against the re-layout path: the same products, so only the order of the fp32 sums may differ (2 k 2^-24 of
+    the terms, which with N(0, 1) operands stays far below 1e-5 of the largest output times sqrt(k)); every output form."""
+    a_bits = workloads.activations_bf16(m, k, seed=510, batch=batch)
+    a_dev = bf16_dev(a_bits).reshape(batch, m, k)
+    w = workloads.weights_f32(k, n, seed=511, batch=b_batch)
+    w_tiles = capi.tilize(bf16_dev(workloads.f32_to_bf16_bits_rne(w)).reshape(b_batch, k, n))
+    bias = bf16_dev(workloads.f32_to_bf16_bits_rne(workloads.normal_tensor((n,), seed=512)))
+    knobs("block", block)
+    call = lambda a=a_dev, layout=capi.ROW_MAJOR, **more: capi.matmul_bf16(a, layout, w_tiles, batch, b_batch, m, k, n, bias=bias, **more)
+    knobs("kernel", "expanded")
+    want = call(out_dtype=torch.float32)
+    knobs("kernel", "bf16 in place")
+    got = call(out_dtype=torch.float32)
+    terms = np.abs(workloads.bf16_bits_to_f32(a_bits).reshape(batch, m, k)) @ np.abs(w.reshape(b_batch, k, n)) + 4.0
+    assert np.all(np.abs((got - want).cpu().numpy()) <= 2.0 * k * 2.0 ** -24 * terms)
+    c16 = call()
+    assert torch.equal(c16.view(torch.int16), got.bfloat16().view(torch.int16))
+    if m % 32 == 0:
+        a_tiles = capi.tilize(a_dev)
+        tiles = call(a_tiles, capi.TILE, c_layout=capi.TILE)
+        assert torch.equal(capi.untilize(tiles, (batch, m, n)).view(torch.int16), c16.view(torch.int16))
+        tiles32 = call(a_tiles, capi.TILE, c_layout=capi.TILE, out_dtype=torch.float32)
+        assert torch.equal(capi.untilize(tiles32, (batch, m, n)), got)
+        for fmt in (BFP8, BFP4):
+            packed = torch.empty(capi.lib().ttmi_tiled_size_bytes(fmt, batch, m, n) // 4, dtype=torch.int32, device="cuda")
+            capi.check(capi.lib().ttmi_matmul_bf16(a_tiles.data_ptr(), capi.TILE, w_tiles.data_ptr(), batch, b_batch, m, k, n, bias.data_ptr(),
+                                                   capi.ACT_NONE, packed.data_ptr(), capi.TILE, fmt, None, 0, torch.cuda.current_stream().cuda_stream))
+            host = oracle.pack_fp32_vec_as_bfp_tiles(fmt, tiles.float().cpu().numpy().reshape(-1), False)
+            assert np.array_equal(packed.cpu().numpy().view(np.uint32), host)
 
 
 @pytest.mark.parametrize("fmt", [BFP8, BFP4])

@@ -149,8 +149,8 @@ def test_matmul_errors(device):
 
 
 def test_matmul_of_two_bfloat16_tensors(device):
-    """ttnn.matmul / ttnn.linear with two bf16 operands (matmul.hpp:39-42): the surface is the same, the weights take the
-    re-layout path of ttmi_matmul_bf16."""
+    """ttnn.matmul / ttnn.linear with two bf16 operands (matmul.hpp:39-42): the surface is that of block-float weights,
+    the GEMM that of ttmi_matmul_bf16."""
     import ttnn
 
     torch.manual_seed(11)

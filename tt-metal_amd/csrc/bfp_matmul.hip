@@ -1239,11 +1239,15 @@ int matmul_bfp(const MatmulArgs &x, hipStream_t st) {
     }
 }
 
-// bf16 x bf16: the weights are brought into the operand layout of the expanding GEMM's second pass (a re-layout instead of
-// an expansion), whatever the number of rows.
+// bf16 x bf16, whatever the number of rows: the kernel that reads the weights as they lie, or (one pass over them, then
+// 256 x 256 blocks) the expanding GEMM's second pass.
 int matmul_bf16(const MatmulArgs &x, hipStream_t st) {
     if (int rc = ttmi_device_status()) return rc;
-    return matmul_bfp_expanded(x, st);
+    if (int rc = validate_expanded(x)) return rc;
+    bool direct = bf16_direct_block(x.batch, x.b_batch, x.m, x.k, x.n) != 0;
+    uint32_t forced;
+    if (knob(TTMI_KNOB_MATMUL_KERNEL, &forced)) direct = forced == 5;
+    return direct ? matmul_bf16_direct(x, st) : matmul_bfp_expanded(x, st);
 }
 
 // c = act(a . b + bias) * (a . b2) in one launch of the 128-column kernel (any number of rows: the weights are streamed

@@ -284,6 +284,21 @@ size_t matmul_expanded_workspace_bytes(uint32_t b_batch, uint32_t k, uint32_t n)
     return (size_t)((uint64_t)b_batch * (k / 32) * groups * GROUP_BYTES);
 }
 
+// What the launches below, and the kernel that reads bf16 weights in place, cannot take.
+int validate_expanded(const MatmulArgs &x) {
+    const uint64_t kt = x.k / 32, groups = ((uint64_t)x.n / 32 + 1) / 2;
+    const uint64_t blocks = (uint64_t)x.batch * ((x.m + 255) / 256) * (((uint64_t)(x.n + 255) / 256 + 7) / 8 * 8), items = (uint64_t)x.b_batch * kt * groups;
+    if (blocks > 0x7fffffffull || items > 0x7fffffffull) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: problem too large for one launch");
+    if ((uint64_t)x.m * x.k * 2 > 0xffffffffull || (uint64_t)((x.m + 31) / 32) * kt * 2048 > 0xffffffffull)
+        return fail(TTMI_ERR_UNSUPPORTED, "matmul: one batch slice of A exceeds 4 GiB");
+    if ((reinterpret_cast<uintptr_t>(x.a) | reinterpret_cast<uintptr_t>(x.b) | reinterpret_cast<uintptr_t>(x.c)) & 15u)
+        return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: a, b and c must be 16-byte aligned");
+    const size_t need = matmul_expanded_workspace_bytes(x.b_batch, x.k, x.n);
+    if (x.workspace && x.workspace_bytes < need) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: workspace of %zu bytes given, %zu needed", x.workspace_bytes, need);
+    if (reinterpret_cast<uintptr_t>(x.workspace) & 255u) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: workspace must be 256-byte aligned");
+    return TTMI_OK;
+}
+
 // x.b: packed block-float tiles (x.b_fmt BFLOAT8_B | BFLOAT4_B) or bf16 tiles (x.b_fmt BFLOAT16)
 int matmul_bfp_expanded(const MatmulArgs &x, hipStream_t st) {
     ExpandedDev p{};
@@ -296,21 +311,12 @@ int matmul_bfp_expanded(const MatmulArgs &x, hipStream_t st) {
     p.c_bfp = x.c_dtype == TTMI_BFLOAT8_B ? 7 : x.c_dtype == TTMI_BFLOAT4_B ? 3 : 0;
     const uint64_t blocks = (uint64_t)x.batch * p.tiles_m * p.tiles_n8 * 8;
     const uint64_t items = (uint64_t)x.b_batch * p.kt * p.groups;
-    if (blocks > 0x7fffffffull || items > 0x7fffffffull) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: problem too large for one launch");
-    if ((uint64_t)x.m * x.k * 2 > 0xffffffffull || (uint64_t)((x.m + 31) / 32) * p.kt * 2048 > 0xffffffffull)
-        return fail(TTMI_ERR_UNSUPPORTED, "matmul: one batch slice of A exceeds 4 GiB");
-    if ((reinterpret_cast<uintptr_t>(x.a) | reinterpret_cast<uintptr_t>(x.b) | reinterpret_cast<uintptr_t>(x.c)) & 15u)
-        return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: a, b and c must be 16-byte aligned");
-    const size_t need = matmul_expanded_workspace_bytes(x.b_batch, x.k, x.n);
-    void *expanded = nullptr;
-    if (x.workspace) {
-        if (x.workspace_bytes < need) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: workspace of %zu bytes given, %zu needed", x.workspace_bytes, need);
-        if (reinterpret_cast<uintptr_t>(x.workspace) & 255u) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: workspace must be 256-byte aligned");
-        expanded = x.workspace;
-    } else {
+    if (int rc = validate_expanded(x)) return rc;
+    void *expanded = x.workspace;
+    if (!expanded) {
         // the library's own buffer, one per stream (launches on one stream run in order, so they can share it)
         bool fresh;
-        if (int rc = scratch_get(SCRATCH_EXPANDED, st, need, &expanded, &fresh)) return rc;
+        if (int rc = scratch_get(SCRATCH_EXPANDED, st, matmul_expanded_workspace_bytes(x.b_batch, x.k, x.n), &expanded, &fresh)) return rc;
     }
     p.w = (const uint8_t *)expanded;
     const uint32_t expand_blocks = (uint32_t)((items + 3) / 4);

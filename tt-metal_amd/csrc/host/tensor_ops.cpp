@@ -454,7 +454,7 @@ Tensor matmul(const Tensor &a, const Tensor &b, bool bcast_batch, const Tensor *
     const bool packed_out = is_block_float(out_dtype);
     const int c_layout = untilize_out ? TTMI_ROW_MAJOR : TTMI_TILE;                                     // bmm_op.cpp:1069
     Buffer c = allocate(packed_out ? storage_bytes(out_dtype, Layout::TILE, {batch_a, m, n}) : c_elements * 2, device);
-    if (b.dtype == DataType::BFLOAT16)      // two bf16 operands: not the tuned path (the weights are re-laid-out on every call), but the same surface
+    if (b.dtype == DataType::BFLOAT16)      // two bf16 operands
         check(ttmi_matmul_bf16(a_tiles.data, TTMI_TILE, b.buffer.data, batch_a, batch_b, m, k, n, bias ? bias_row.data : nullptr, activation, c.data,
                                c_layout, packed_out ? (int)out_dtype : TTMI_BFLOAT16, nullptr, 0, stream_of(device)));
     else if (a_in_kernel)
