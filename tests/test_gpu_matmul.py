@@ -737,6 +737,58 @@ def test_bf16_weights(batch, b_batch, m, k, n):
     assert torch.equal(again.view(torch.int16), c16.view(torch.int16))
 
 
+def check_on_device(c, a, w, k):
+    """The fp32 accumulation bound (2 k 2^-24 of the terms) on an fp32 result, evaluated in float64 on the GPU."""
+    ref, terms = a.double() @ w.double(), a.double().abs() @ w.double().abs()
+    assert bool(((c.double() - ref).abs() <= 2.0 * k * 2.0 ** -24 * terms + 1e-37).all())
+
+
+@pytest.mark.parametrize("fmt", [BFP8, BFP4])
+# blocks of 256 x 256: one in two k ranges (of 16 and 17 steps); four in four, on XCDs with and without one; 259 = 32 or 33 per XCD,
+# the 33rd cut in two; 264, the same on every XCD
+@pytest.mark.parametrize("batch,m,k,n", [(1, 40, 1056, 96), (2, 260, 2080, 256), (1, 7 * 256 - 32, 1024, 37 * 256 - 32), (1, 8448, 1024, 2048)])
+def test_k_ranges_of_the_expanding_gemm(oracle, batch, m, k, n, fmt, knobs):
+    """Blocks cut into k ranges (scratch of the library) against float64 and against the same GEMM on a caller's workspace that
+    holds the weights alone, where nothing is cut; every output form; a workspace with room for the sums gives the same bits."""
+    knobs("kernel", "expanded")
+    a = bf16_dev(workloads.activations_bf16(m, k, seed=520, batch=batch)).reshape(batch, m, k)
+    w = torch.from_numpy(workloads.weights_f32(k, n, seed=521, batch=batch)).cuda().reshape(batch, k, n)
+    words = capi.pack_tensor(fmt, w)
+    w = capi.unpack_tensor(fmt, words, (batch, k, n))
+    bias = bf16_dev(workloads.f32_to_bf16_bits_rne(workloads.normal_tensor((n,), seed=522)))
+    need = capi.lib().ttmi_matmul_bfp_workspace_bytes(batch, m, k, n, fmt)
+    call = lambda a=a, layout=capi.ROW_MAJOR, **more: capi.matmul_bfp(a, layout, words, fmt, batch, batch, m, k, n, **more)
+    c = call(out_dtype=torch.float32)
+    plain = call(out_dtype=torch.float32, workspace=torch.empty(need, dtype=torch.uint8, device="cuda"))
+    for s in range(batch):
+        check_on_device(c[s], a[s], w[s], k)
+        check_on_device(plain[s], a[s], w[s], k)
+    roomy = torch.full((need + (80 << 20),), 0x5A, dtype=torch.uint8, device="cuda")
+    assert torch.equal(call(out_dtype=torch.float32, workspace=roomy), c)
+    biased = call(bias=bias, activation=capi.ACT_RELU)
+    assert torch.equal(biased.view(torch.int16), torch.relu(c + bias.float()).bfloat16().view(torch.int16))
+    if m % 32 == 0:
+        tiles = call(capi.tilize(a), capi.TILE, c_layout=capi.TILE)
+        assert torch.equal(capi.untilize(tiles, (batch, m, n)).view(torch.int16), c.bfloat16().view(torch.int16))
+        packed = call(capi.tilize(a), capi.TILE, c_layout=capi.TILE, out_bfp=fmt)
+        host = oracle.pack_fp32_vec_as_bfp_tiles(fmt, tiles.float().cpu().numpy().reshape(-1), False)
+        assert np.array_equal(packed.cpu().numpy().view(np.uint32), host)
+
+
+@pytest.mark.parametrize("batch,m,k,n", [(8, 384, 1024, 4096), (5, 333, 512, 2112), (64, 32, 1024, 4096)])
+def test_slices_that_share_their_weights(batch, m, k, n):
+    """Slices with common weights, multiplied as the rows of one GEMM where that is better: float64, dense and tiles alike."""
+    a = bf16_dev(workloads.activations_bf16(m, k, seed=530, batch=batch)).reshape(batch, m, k)
+    words = capi.pack_tensor(BFP8, torch.from_numpy(workloads.weights_f32(k, n, seed=531)).cuda().reshape(1, k, n))
+    w = capi.unpack_tensor(BFP8, words, (1, k, n))[0]
+    c = capi.matmul_bfp(a, capi.ROW_MAJOR, words, BFP8, batch, 1, m, k, n, out_dtype=torch.float32)
+    for s in range(batch):
+        check_on_device(c[s], a[s], w, k)
+    if m % 32 == 0:
+        tiles = capi.matmul_bfp(capi.tilize(a), capi.TILE, words, BFP8, batch, 1, m, k, n, c_layout=capi.TILE)
+        assert torch.equal(capi.untilize(tiles, (batch, m, n)).view(torch.int16), c.bfloat16().view(torch.int16))
+
+
 @pytest.mark.parametrize("block", [64, 128])
 @pytest.mark.parametrize("batch,b_batch,m,k,n", [(1, 1, 1, 32, 32), (1, 1, 33, 64, 96), (2, 2, 127, 96, 160), (3, 1, 160, 128, 288), (17, 17, 64, 160, 64)])
 def test_bf16_weights_read_in_place(oracle, batch, b_batch, m, k, n, block, knobs):

@@ -1140,6 +1140,15 @@ int matmul_bfp_wide(const MatmulArgs &x, hipStream_t st) { return launch_streami
 // on (two or more 256-row blocks share every weight) the weights are expanded to bf16 once and a plain bf16 GEMM follows.
 // The test entry point can force a kernel (TTMI_KNOB_MATMUL_KERNEL).
 enum class Kernel { Stream = 1, Wide = 2, Tile = 3, Expanded = 4 };
+static double streamed_estimate(uint32_t batch, uint32_t m, uint32_t k, uint32_t n, int b_fmt) {
+    const double weights = (double)k * n * (b_fmt == TTMI_BFLOAT8_B ? 1.0625 : 0.8);     // BFLOAT4_B: half the bytes, the same instructions
+    const double sets = (double)batch * (((m + 31) / 32 + 1) / 2);
+    return 8.0 + sets * weights / 4.7e6;
+}
+static double tiled_estimate(uint32_t batch, uint32_t m, uint32_t k, uint32_t n) {
+    const double blocks = (double)batch * ((m + 127) / 128) * ((n + 255) / 256);
+    return std::ceil(blocks / 256.0) * (k / 32) * 0.78;
+}
 static Kernel choose_kernel(uint32_t batch, uint32_t m, uint32_t k, uint32_t n, int b_fmt, bool c_bfp) {
     uint32_t forced;
     if (knob(TTMI_KNOB_MATMUL_KERNEL, &forced) && forced >= 1 && forced <= 4) return (Kernel)forced;
@@ -1151,16 +1160,13 @@ static Kernel choose_kernel(uint32_t batch, uint32_t m, uint32_t k, uint32_t n, 
         // against 102 (tiled) and 85 (expanded); [128, 14336] x [14336, 4096] 34 against 331 and 264; [256, 4096] x
         // [4096, 14336] 54 against 103 and 105; [448, 4544] x [4544, 18176] 138 against 229 and 130; 12 x [384, 1024] x
         // [1024, 1024] 29.5 against 24.8 (the 384-row kernel).  The estimates below reproduce those within 15 %.
-        const double k_tiles = k / 32, weights = (double)k * n * (b_fmt == TTMI_BFLOAT8_B ? 1.0625 : 0.8);     // BFLOAT4_B: half the bytes, the same instructions
-        const double sets = (double)batch * (((m + 31) / 32 + 1) / 2);
-        const double streamed_us = 8.0 + sets * weights / 4.7e6;
+        const double k_tiles = k / 32, streamed_us = streamed_estimate(batch, m, k, n, b_fmt);
         double blocked_us;
         if (m >= 512) {
             const double blocks = (double)batch * ((m + 255) / 256) * ((n + 255) / 256);
             blocked_us = 4.0 + (double)k * n * 3.0625 / 6.0e6 + std::ceil(blocks / 256.0) * k_tiles * 0.72;      // expansion pass + bf16 GEMM
         } else {
-            const double blocks = (double)batch * ((m + 127) / 128) * ((n + 255) / 256);
-            blocked_us = std::ceil(blocks / 256.0) * k_tiles * 0.78;
+            blocked_us = tiled_estimate(batch, m, k, n);
         }
         if (streamed_us < 0.9 * blocked_us) return Kernel::Wide;
         return m >= 512 ? Kernel::Expanded : Kernel::Tile;
@@ -1178,6 +1184,36 @@ static Kernel choose_kernel(uint32_t batch, uint32_t m, uint32_t k, uint32_t n, 
         one_round_of_groups((uint64_t)batch * ((n / 32 + GROUP_TILES - 1) / GROUP_TILES)))
         return Kernel::Stream;
     return m <= 32 || ((m + 31) / 32) % 2 == 0 || c_bfp || k >= n ? Kernel::Wide : Kernel::Stream;
+}
+
+// With scratch of the library's own the expanding GEMM can also cut k ranges (a caller's workspace, sized by
+// matmul_workspace_bytes, has no room for the partial sums), which is what outputs of few blocks and last rounds on a part
+// of the chip need.  Measured, same box: [1000, 14336] x [14336, 4096] BFLOAT4_B, 64 blocks, 152 us in four k ranges against
+// 205 streamed; [200, 4096] x [4096, 14336] and [300, 16384] x [16384, 16384] are better streamed (63 us, 310 us), as estimated.
+static Kernel choose_kernel_own_scratch(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, int b_fmt, bool c_bfp) {
+    const Kernel kernel = choose_kernel(batch, m, k, n, b_fmt, c_bfp);
+    uint32_t forced;
+    if (m < 128 || kernel == Kernel::Expanded || knob(TTMI_KNOB_MATMUL_KERNEL, &forced)) return kernel;
+    const double now = kernel == Kernel::Tile ? tiled_estimate(batch, m, k, n) : streamed_estimate(batch, m, k, n, b_fmt);
+    const double expanded = matmul_expanded_estimate(batch, b_batch, m, k, n, b_fmt == TTMI_BFLOAT8_B ? 1.0625 : 0.5625);
+    return expanded < 0.95 * now ? Kernel::Expanded : kernel;
+}
+
+// Slices that share their weights are one GEMM of all their rows: [batch, m, k] lies in memory as [1, batch m, k] does, dense
+// or in whole tiles (TILE layouts have m % 32 == 0), and blocks of rows need not end with a slice.  Taken where the rows
+// together go to the expanding GEMM and it is the better one: 8 x [384, 1024] x [1024, 4096] 39 us against 67 slice by slice
+// (tiled).  Not for streamed shapes, whose slices share the weights through the caches: 2 x [32, 4096] x [4096, 4096] 13.6
+// against 10.2 us as they are.
+static bool fold_batch(const MatmulArgs &x, bool c_bfp) {
+    const uint64_t rows = (uint64_t)x.batch * x.m;
+    uint32_t forced;
+    if (x.b_batch != 1 || x.batch == 1 || rows * x.k * 2 > 0xffffffffull || rows > 0x7fffff00ull || knob(TTMI_KNOB_MATMUL_KERNEL, &forced)) return false;
+    if (choose_kernel_own_scratch(1, 1, (uint32_t)rows, x.k, x.n, x.b_fmt, c_bfp) != Kernel::Expanded) return false;
+    const double bytes = x.b_fmt == TTMI_BFLOAT8_B ? 1.0625 : 0.5625;
+    const Kernel as_is = choose_kernel_own_scratch(x.batch, 1, x.m, x.k, x.n, x.b_fmt, c_bfp);
+    const double slices = as_is == Kernel::Expanded ? matmul_expanded_estimate(x.batch, 1, x.m, x.k, x.n, bytes)
+                        : as_is == Kernel::Tile ? tiled_estimate(x.batch, x.m, x.k, x.n) : streamed_estimate(x.batch, x.m, x.k, x.n, x.b_fmt);
+    return matmul_expanded_estimate(1, 1, (uint32_t)rows, x.k, x.n, bytes) < slices;
 }
 
 size_t matmul_gated_workspace_bytes(uint32_t batch, uint32_t m, uint32_t k, uint32_t n) {
@@ -1204,7 +1240,7 @@ size_t matmul_workspace_bytes(uint32_t batch, uint32_t m, uint32_t k, uint32_t n
 void matmul_plan(uint32_t batch, uint32_t m, uint32_t k, uint32_t n, int b_fmt, bool a_or_c_bfp, uint32_t out[4]) {
     out[0] = out[1] = out[2] = out[3] = 0;
     if (!batch || !m || !k || !n) return;
-    const Kernel kernel = choose_kernel(batch, m, k, n, b_fmt, a_or_c_bfp);
+    const Kernel kernel = choose_kernel_own_scratch(batch, batch, m, k, n, b_fmt, a_or_c_bfp);
     out[0] = (uint32_t)kernel;
     if (kernel != Kernel::Wide && kernel != Kernel::Stream) return;
     const bool wide = kernel == Kernel::Wide;
@@ -1220,14 +1256,19 @@ bool matmul_takes_bfp_activations(uint32_t batch, uint32_t m, uint32_t k, uint32
     return batch && m == 32 && k && n && choose_kernel(batch, m, k, n, b_fmt, true) == Kernel::Wide;
 }
 
-int matmul_bfp(const MatmulArgs &x, hipStream_t st) {
+int matmul_bfp(const MatmulArgs &asked, hipStream_t st) {
+    MatmulArgs x = asked;
     // what an earlier launch on this device has reported (a wait for partial sums that gave up) surfaces here
     if (!x.no_alloc || error_word_if_exists(nullptr, nullptr))
         if (int rc = ttmi_device_status()) return rc;
     // every kernel but the 64-column one packs a block-float output in its epilogue (choose_kernel keeps that one out of it)
     const bool c_bfp = x.c_dtype == TTMI_BFLOAT8_B || x.c_dtype == TTMI_BFLOAT4_B;
     const bool a8 = x.a_dtype == TTMI_BFLOAT8_B;      // block-float activations: the 128-column kernel alone takes them
-    const Kernel kernel = choose_kernel(x.batch, x.m, x.k, x.n, x.b_fmt, c_bfp || a8);
+    // (the workspace query answers for the slices as they are, so a caller's workspace serves those)
+    const bool own_scratch = !x.workspace && !x.no_alloc;
+    if (own_scratch && !a8 && fold_batch(x, c_bfp)) { x.m *= x.batch; x.batch = 1; }
+    const Kernel kernel = own_scratch ? choose_kernel_own_scratch(x.batch, x.b_batch, x.m, x.k, x.n, x.b_fmt, c_bfp || a8)
+                                      : choose_kernel(x.batch, x.m, x.k, x.n, x.b_fmt, c_bfp || a8);
     if (a8 && !matmul_takes_bfp_activations(x.batch, x.m, x.k, x.n, x.b_fmt))
         return fail(TTMI_ERR_UNSUPPORTED, "matmul: block-float activations are taken by the one-band streaming kernel only, which this shape does "
                     "not go to (ttmi_matmul_bfp_ab_supported): expand them with ttmi_typecast_tiles first");

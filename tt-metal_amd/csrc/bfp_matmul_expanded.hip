@@ -15,7 +15,8 @@
 #include <stdint.h>
 #include <stdlib.h>
 
-#include <mutex>
+#include <algorithm>
+#include <cmath>
 
 #include "bfp_dequant.h"
 #include "ttmi_internal.h"
@@ -136,11 +137,27 @@ struct ExpandedDev {
     const uint16_t *bias;    // bf16 [n] or null
     uint8_t *c;
     uint32_t batch, b_batch, m, k, n;
-    uint32_t kt, nt, groups, tiles_m, tiles_n, tiles_n8;
+    uint32_t kt, nt, groups, tiles_m, tiles_n;
+    uint32_t per_xcd, extra; // blocks of C per XCD: one more for the first `extra` of the 8
+    uint32_t whole, tail;    // of those, done in one piece | cut into `split` k ranges
+    uint32_t split;
+    float *parts;            // [tail block][k range] x PART_FLOATS partial sums
     float unscale;
     int a_tiled, c_tiled, c_f32;
     int c_bfp;               // 0, or the mantissa bits (7 | 3) of a block-float output in TILE layout
 };
+
+constexpr uint32_t PART_FLOATS = 256 * 256;
+
+// block of C number `local` of an XCD; false when this XCD has no such block
+__device__ __forceinline__ bool expanded_block(const ExpandedDev &p, uint32_t xcd, uint32_t local, uint32_t &tm, uint32_t &tn, uint32_t &bb) {
+    if (local >= p.per_xcd + (xcd < p.extra ? 1u : 0u)) return false;
+    uint32_t idx = xcd * p.per_xcd + min(xcd, p.extra) + local;
+    tm = idx % p.tiles_m; idx /= p.tiles_m;
+    tn = idx % p.tiles_n;
+    bb = idx / p.tiles_n;
+    return true;
+}
 
 constexpr int EXP_STAGES = 4;
 
@@ -148,8 +165,12 @@ constexpr int EXP_STAGES = 4;
 // the 256 x 256 block: 4 x 2 accumulator blocks of 32 x 32.
 //   LDS     ring of EXP_STAGES stages [A: 256 rows x 64 B, chunks XOR-swizzled][B: 4 column groups as they lie in the
 //           workspace, 16 KB], both filled by direct global->LDS loads (4 per wavefront and step)
-//   blocks  workgroup i runs on XCD i % 8.  An XCD takes every 8th 256-column block and all row blocks of it at the
-//           same time, so a weight is fetched into one L2 only and A (small) is what every L2 re-reads.
+//   blocks  workgroup i runs on XCD i % 8.  An XCD takes a contiguous run of blocks, row blocks first, so that all row
+//           blocks of a column block run there at the same time: a weight is fetched into one or two L2s only and A
+//           (small) is what every L2 re-reads.
+//   k       the blocks that would be a last round on part of an XCD's 32 CUs (all of them, when there are fewer) are cut
+//           into `split` k ranges, one workgroup each, whose sums go to memory as they lie in the registers and are
+//           added, in order, by reduce_parts_kernel
 //   step s  wait until everything requested before the previous step has landed (step s+1 complete in LDS), barrier,
 //           then per 16-row slab 8 MFMAs, each followed by one LDS read of the following slab's operands (the first
 //           slab of step s+1 at the end) or one request for step s+3.
@@ -165,14 +186,17 @@ __global__ __launch_bounds__(512, 1) void matmul_expanded_kernel(const ExpandedD
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wc = wave & 3, wr = wave >> 2;
     const int c = lane & 31, kh = lane >> 5;
-    const uint32_t last = p.kt - 1;
-
-    uint32_t idx = blockIdx.x;
-    const uint32_t xcd = idx & 7; idx >>= 3;
-    const uint32_t tm = idx % p.tiles_m; idx /= p.tiles_m;
-    const uint32_t tn = (idx % p.tiles_n8) * 8 + xcd;
-    const uint32_t bb = idx / p.tiles_n8;
-    if (tn >= p.tiles_n) return;                                         // the whole workgroup, before any barrier
+    const uint32_t xcd = blockIdx.x & 7, item = blockIdx.x >> 3;
+    uint32_t local = item, part = 0, first = 0, end = p.kt, tm, tn, bb;
+    const bool partial = item >= p.whole && p.split > 1;
+    if (partial) {                                                       // neighbours take different blocks and the same k range
+        part = (item - p.whole) / p.tail;
+        local = p.whole + (item - p.whole) % p.tail;
+        first = p.kt * part / p.split;
+        end = p.kt * (part + 1) / p.split;
+    }
+    if (!expanded_block(p, xcd, local, tm, tn, bb)) return;              // the whole workgroup, before any barrier
+    const uint32_t last = end - 1;
     const uint32_t m0 = tm * 256;
 
     // ---- requests of this wavefront: rows 32w .. 32w+31 of A, KB 2w, 2w+1 of the block's 16 KB of B -------------
@@ -230,11 +254,11 @@ __global__ __launch_bounds__(512, 1) void matmul_expanded_kernel(const ExpandedD
             for (int r = 0; r < 16; ++r) acc[rb][cb][r] = 0.f;
 
     bf16x8 a0[RB], b0[CB], a1[RB], b1[CB], a2[RB], b2[CB];
-    request(0); request(1); request(2);
+    request(first); request(first + 1); request(first + 2);
     wait_vmcnt<VM_PER_STEP>();                 // steps 0 and 1 have landed (ours)
     __builtin_amdgcn_s_barrier();              // everybody's
 #pragma unroll
-    for (int j = 0; j < 6; ++j) read_operand(0, 0, j, a0, b0);
+    for (int j = 0; j < 6; ++j) read_operand(first, 0, j, a0, b0);
 
     // Between two MFMAs a wavefront issues at most one LDS read or one request (order of the reads: what the next slab
     // needs first), so that the matrix pipe never waits for a burst of them.  The operands of the next step's first
@@ -261,22 +285,99 @@ __global__ __launch_bounds__(512, 1) void matmul_expanded_kernel(const ExpandedD
         }
         asm volatile("" ::: "memory");         // the requests stay in this step
     };
-    uint32_t kstep = 0;
+    uint32_t kstep = first;
 #pragma unroll 1
-    for (; kstep + 2 <= p.kt; kstep += 2) {
+    for (; kstep + 2 <= end; kstep += 2) {
         step_body(kstep, a0, b0, a2, b2);
         step_body(kstep + 1, a2, b2, a0, b0);
     }
-    if (kstep < p.kt) step_body(kstep, a0, b0, a2, b2);
+    if (kstep < end) step_body(kstep, a0, b0, a2, b2);
     wait_vmcnt<0>();                           // requests past the end have landed,
     __builtin_amdgcn_s_waitcnt(0xC07F);
     __builtin_amdgcn_s_barrier();              // and nobody reads operands any more: the ring becomes 8 x 16 KB of staging
+
+    if (partial) {
+        f32x4 *to = reinterpret_cast<f32x4 *>(p.parts + ((uint64_t)(xcd * p.tail + local - p.whole) * p.split + part) * PART_FLOATS) + wave * 2048 + lane;
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+#pragma unroll
+            for (int cb = 0; cb < CB; ++cb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    to[((rb * 2 + cb) * 4 + i) * 64] = f32x4{acc[rb][cb][4 * i], acc[rb][cb][4 * i + 1], acc[rb][cb][4 * i + 2], acc[rb][cb][4 * i + 3]};
+        return;
+    }
 
     StoreTarget o;
     o.c = p.c; o.bias = p.bias; o.m = p.m; o.n = p.n; o.nt = p.nt; o.slice = bb;
     o.row0 = m0 + wr * 128; o.nt0 = (tn * 4 + wc) * 2;
     o.unscale = p.unscale; o.c_tiled = p.c_tiled; o.c_f32 = p.c_f32; o.c_bfp = p.c_bfp;
     store_wave_part<ACT>(acc, o, lds + wave * 16384, lane);
+}
+
+// Adds the k ranges of the blocks that were cut, in order, and stores C.  One wavefront per 32 x 64 part of a block, the sums
+// 16 bytes per lane as the GEMM left them: bound by reading them back (out of the Infinity Cache, where they have just been put).
+template <int ACT>
+__global__ __launch_bounds__(256) void reduce_parts_kernel(const ExpandedDev p) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[4 * 4096];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t item = blockIdx.x * 4 + wave, rb = item & 3, w = (item >> 2) & 7, block = item >> 5;
+    const uint32_t xcd = block / p.tail, i = block % p.tail;
+    uint32_t tm, tn, bb;
+    if (!expanded_block(p, xcd, p.whole + i, tm, tn, bb)) return;        // no barrier in this kernel
+    const uint32_t row0 = tm * 256 + (w >> 2) * 128 + rb * 32;
+    if (row0 >= p.m) return;
+    const f32x4 *from = reinterpret_cast<const f32x4 *>(p.parts + (uint64_t)block * p.split * PART_FLOATS) + w * 2048 + rb * 512 + lane;
+    f32x16 acc[1][2];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+        const f32x4 v = from[j * 64];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[0][j >> 2][(j & 3) * 4 + e] = v[e];
+    }
+    for (uint32_t part = 1; part < p.split; ++part) {
+        from += PART_FLOATS / 4;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            const f32x4 v = from[j * 64];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[0][j >> 2][(j & 3) * 4 + e] += v[e];
+        }
+    }
+    StoreTarget o;
+    o.c = p.c; o.bias = p.bias; o.m = p.m; o.n = p.n; o.nt = p.nt; o.slice = bb;
+    o.row0 = row0; o.nt0 = (tn * 4 + (w & 3)) * 2;
+    o.unscale = p.unscale; o.c_tiled = p.c_tiled; o.c_f32 = p.c_f32; o.c_bfp = p.c_bfp;
+    store_wave_part<ACT>(acc, o, lds + wave * 4096, lane);
+}
+
+// How the blocks of C are dealt out, and the estimated time of the whole product.  A k tile row of a 256 x 256 block takes
+// 0.72 us; expanding moves 2 bytes per weight out and the packed ones in; a cut block's sums are written and read once.
+// Measured (kernel trace, one MI355X): [2048, 4544] x [4544, 18176], 568 blocks = two rounds and 7 of 32 places per XCD, the
+// last round in 4 k ranges: 275 us (315 once the chip is hot) + 13 for the sums, against 324 (358) in three rounds;
+// [1000, 14336] x [14336, 4096], 64 blocks in 4 k ranges on 256 CUs: 97 + 14 us.
+struct ExpandedPlan { uint64_t per_xcd; uint32_t extra, whole, tail, split; size_t parts_bytes; double us; };
+static ExpandedPlan plan_expanded(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, double bytes_per_weight, bool may_split) {
+    constexpr uint32_t CUS = 32;                                          // per XCD
+    constexpr uint32_t LEAST_STEPS = 16;                                  // a k range below that is mostly start-up and hand-over
+    const uint64_t blocks = (uint64_t)batch * ((m + 255) / 256) * ((n + 255) / 256);
+    const uint32_t kt = k / 32;
+    ExpandedPlan e{};
+    e.per_xcd = blocks / 8; e.extra = (uint32_t)(blocks % 8);
+    const uint64_t most = e.per_xcd + (e.extra ? 1 : 0);
+    e.tail = (uint32_t)(most % CUS);
+    e.split = may_split && e.tail ? std::min(CUS / e.tail, kt / LEAST_STEPS) : 1;
+    if (e.split < 2) { e.split = 1; e.tail = 0; }
+    e.whole = (uint32_t)(most - e.tail);
+    const uint64_t cut = e.tail ? (blocks > 8ull * e.whole ? blocks - 8ull * e.whole : 0) : 0;
+    e.parts_bytes = e.tail ? (size_t)8 * e.tail * e.split * PART_FLOATS * 4 : 0;
+    const double rounds = std::ceil(e.whole / (double)CUS) + (e.tail ? 1.0 / e.split : 0.0);
+    e.us = 8.0 + (double)b_batch * k * n * (bytes_per_weight + 2.0) / 5.5e6 + rounds * kt * 0.72 + (e.tail ? 3.0 + (double)cut * e.split * PART_FLOATS * 8 / 5.0e6 : 0.0);
+    return e;
+}
+double matmul_expanded_estimate(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, double bytes_per_weight) {
+    return plan_expanded(batch, b_batch, m, k, n, bytes_per_weight, true).us;
 }
 
 size_t matmul_expanded_workspace_bytes(uint32_t b_batch, uint32_t k, uint32_t n) {
@@ -299,25 +400,36 @@ int validate_expanded(const MatmulArgs &x) {
     return TTMI_OK;
 }
 
+template <int ACT> static void launch_expanded(const ExpandedDev &p, uint32_t blocks, hipStream_t st) {
+    hipLaunchKernelGGL((matmul_expanded_kernel<ACT>), dim3(blocks), dim3(512), 0, st, p);
+    if (p.tail) hipLaunchKernelGGL((reduce_parts_kernel<ACT>), dim3(8 * p.tail * 8), dim3(256), 0, st, p);
+}
+
 // x.b: packed block-float tiles (x.b_fmt BFLOAT8_B | BFLOAT4_B) or bf16 tiles (x.b_fmt BFLOAT16)
 int matmul_bfp_expanded(const MatmulArgs &x, hipStream_t st) {
     ExpandedDev p{};
     p.a = (const uint8_t *)x.a; p.bias = (const uint16_t *)x.bias; p.c = (uint8_t *)x.c;
     p.batch = x.batch; p.b_batch = x.b_batch; p.m = x.m; p.k = x.k; p.n = x.n;
     p.kt = x.k / 32; p.nt = x.n / 32; p.groups = (p.nt + 1) / 2;
-    p.tiles_m = (x.m + 255) / 256; p.tiles_n = (x.n + 255) / 256; p.tiles_n8 = (p.tiles_n + 7) / 8;
+    p.tiles_m = (x.m + 255) / 256; p.tiles_n = (x.n + 255) / 256;
     p.unscale = x.b_fmt == TTMI_BFLOAT8_B ? Wfmt<7>::unscale : x.b_fmt == TTMI_BFLOAT4_B ? Wfmt<3>::unscale : 1.0f;
     p.a_tiled = x.a_layout == TTMI_TILE; p.c_tiled = x.c_layout == TTMI_TILE; p.c_f32 = x.c_dtype == TTMI_FLOAT32;
     p.c_bfp = x.c_dtype == TTMI_BFLOAT8_B ? 7 : x.c_dtype == TTMI_BFLOAT4_B ? 3 : 0;
-    const uint64_t blocks = (uint64_t)x.batch * p.tiles_m * p.tiles_n8 * 8;
     const uint64_t items = (uint64_t)x.b_batch * p.kt * p.groups;
     if (int rc = validate_expanded(x)) return rc;
+    const size_t weights_bytes = (matmul_expanded_workspace_bytes(x.b_batch, x.k, x.n) + 255) & ~(size_t)255;
+    ExpandedPlan e = plan_expanded(x.batch, x.b_batch, x.m, x.k, x.n, 0, true);
     void *expanded = x.workspace;
     if (!expanded) {
         // the library's own buffer, one per stream (launches on one stream run in order, so they can share it)
         bool fresh;
-        if (int rc = scratch_get(SCRATCH_EXPANDED, st, matmul_expanded_workspace_bytes(x.b_batch, x.k, x.n), &expanded, &fresh)) return rc;
+        if (int rc = scratch_get(SCRATCH_EXPANDED, st, weights_bytes + e.parts_bytes, &expanded, &fresh)) return rc;
+    } else if (x.workspace_bytes < weights_bytes + e.parts_bytes) {
+        e = plan_expanded(x.batch, x.b_batch, x.m, x.k, x.n, 0, false);      // a caller's workspace has to hold the weights; partial sums only if they fit
     }
+    p.per_xcd = (uint32_t)e.per_xcd; p.extra = e.extra; p.whole = e.whole; p.tail = e.tail; p.split = e.split;
+    p.parts = reinterpret_cast<float *>((uint8_t *)expanded + weights_bytes);
+    const uint32_t blocks = 8 * (e.whole + e.tail * e.split);
     p.w = (const uint8_t *)expanded;
     const uint32_t expand_blocks = (uint32_t)((items + 3) / 4);
     if (x.b_fmt == TTMI_BFLOAT8_B)
@@ -328,10 +440,10 @@ int matmul_bfp_expanded(const MatmulArgs &x, hipStream_t st) {
         hipLaunchKernelGGL(relayout_bf16_kernel, dim3(expand_blocks), dim3(256), 0, st, (const uint8_t *)x.b, (uint8_t *)expanded, p.nt, p.groups, (uint32_t)items);
     if (int rc = check_launch("expand_kernel")) return rc;
     switch (x.activation) {
-        case TTMI_ACT_RELU: hipLaunchKernelGGL((matmul_expanded_kernel<TTMI_ACT_RELU>), dim3((uint32_t)blocks), dim3(512), 0, st, p); break;
-        case TTMI_ACT_GELU: hipLaunchKernelGGL((matmul_expanded_kernel<TTMI_ACT_GELU>), dim3((uint32_t)blocks), dim3(512), 0, st, p); break;
-        case TTMI_ACT_SILU: hipLaunchKernelGGL((matmul_expanded_kernel<TTMI_ACT_SILU>), dim3((uint32_t)blocks), dim3(512), 0, st, p); break;
-        default: hipLaunchKernelGGL((matmul_expanded_kernel<TTMI_ACT_NONE>), dim3((uint32_t)blocks), dim3(512), 0, st, p); break;
+        case TTMI_ACT_RELU: launch_expanded<TTMI_ACT_RELU>(p, blocks, st); break;
+        case TTMI_ACT_GELU: launch_expanded<TTMI_ACT_GELU>(p, blocks, st); break;
+        case TTMI_ACT_SILU: launch_expanded<TTMI_ACT_SILU>(p, blocks, st); break;
+        default: launch_expanded<TTMI_ACT_NONE>(p, blocks, st); break;
     }
     return check_launch("matmul_expanded_kernel");
 }

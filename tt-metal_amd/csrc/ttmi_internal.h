@@ -96,6 +96,7 @@ int matmul_bfp_expanded(const MatmulArgs &args, hipStream_t st);   // expand the
 int matmul_bf16_direct(const MatmulArgs &args, hipStream_t st);    // bf16 weights read as they lie, no pass over them first
 uint32_t bf16_direct_block(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n);    // the block edge a shape gets there, 0: not for it
 int validate_expanded(const MatmulArgs &args);
+double matmul_expanded_estimate(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, double bytes_per_weight);   // us, k ranges cut where that helps
 size_t matmul_expanded_workspace_bytes(uint32_t b_batch, uint32_t k, uint32_t n);
 
 }  // namespace ttmi
