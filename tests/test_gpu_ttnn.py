@@ -309,3 +309,41 @@ def test_untilize_out_gives_the_tile_result_row_major(device, m):
     assert torch.equal(rows.cpu().to_torch().view(torch.int16), ttl.tensor.bmm(ta, twb).cpu().to(ttl.tensor.Layout.ROW_MAJOR).to_torch().view(torch.int16))
     with pytest.raises(RuntimeError, match="output_dtype == DataType::BFLOAT16"):
         ttl.operations.primary.matmul(ta, tw, output_dtype=ttl.tensor.DataType.BFLOAT8_B, untilize_out=True)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1000, 4544), (3, 1, 333, 1111), (2, 2, 64, 16384), (1, 1, 96, 16416), (3, 1, 3001, 3201), (7, 1, 120, 16384)])
+@pytest.mark.parametrize("name,source", [("bfloat8_b", "fp32"), ("bfloat4_b", "fp32"), ("bfloat4_b", "bf16")])
+def test_large_tensors_from_and_to_host_memory(device, shape, name, source):
+    """Tensors large enough to go through pinned slots in bands of tile rows (ragged rows and columns, slices that end inside a
+    band, rows of exactly a slot's 32nd part and one tile longer, which go in one piece): the codes and the values that the
+    kernels give for the whole tensor on the device; from two threads at once, of which one has to go without the slots."""
+    import threading
+
+    import ttnn
+    from ttmi import capi
+
+    dtype, fmt = getattr(ttnn, name), {"bfloat8_b": capi.BFLOAT8_B, "bfloat4_b": capi.BFLOAT4_B}[name]
+    host = torch.randn(shape, generator=torch.Generator().manual_seed(7))
+    host = host if source == "fp32" else host.bfloat16()
+    want = capi.pack_tensor(fmt, host.cuda())
+    back = capi.unpack_tensor(fmt, want, shape).cpu()
+    results = [None, None]
+
+    def one(i):
+        t = ttnn.from_torch(host, dtype=dtype, layout=ttnn.TILE_LAYOUT, device=device)
+        results[i] = (t._buf.view(torch.int32).clone(), ttnn.to_torch(t))
+
+    one(0)
+    threads = [threading.Thread(target=one, args=(i,)) for i in range(2)]
+    for codes, values in [results[0]]:
+        assert torch.equal(codes.cpu(), want.cpu()) and torch.equal(values, back)
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for codes, values in results:
+        assert torch.equal(codes.cpu(), want.cpu()) and torch.equal(values, back)
+    on_host = ttnn.from_torch(host, dtype=dtype, layout=ttnn.TILE_LAYOUT)
+    assert torch.equal(ttnn.to_torch(on_host), back)
+    pinned = ttnn.from_torch(host.pin_memory(), dtype=dtype, layout=ttnn.TILE_LAYOUT, device=device)
+    assert torch.equal(pinned._buf.view(torch.int32).cpu(), want.cpu())
