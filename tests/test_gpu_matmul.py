@@ -737,6 +737,24 @@ def test_bf16_weights(batch, b_batch, m, k, n):
     assert torch.equal(again.view(torch.int16), c16.view(torch.int16))
 
 
+@pytest.mark.parametrize("kernel", ["stream", "wide", "tile", "expanded"])
+def test_gelu_over_its_range(kernel, knobs):
+    """GELU of the values that a product with the identity gives in fp32 (the same call without activation says which: the streaming
+    kernels' sums pass through neighbours of the weights, so they need not be the inputs bit for bit), where its two forms of
+    erf meet (|x| = sqrt(2)), where erf reaches 1 and far beyond.  Bound: erf to 7.1e-8, its argument to 2^-24 (x d erf / dx <= 0.5 in relative terms), the sum
+    1 + erf and two products to 2^-24 each: less than 2^-21 |x| in all."""
+    knobs("kernel", kernel)
+    x = torch.cat([torch.linspace(-9, 9, 3000), torch.linspace(-1.43, -1.40, 500), torch.linspace(1.40, 1.43, 500),
+                   torch.tensor([0.0, -0.0, 1e-30, -1e-30, 40.0, -40.0, 1e4, -1e4])])
+    x = torch.nn.functional.pad(x, (0, -len(x) % 1024)).reshape(-1, 32).bfloat16().cuda()
+    m = x.shape[0]
+    words = capi.pack_tensor(BFP8, torch.eye(32, device="cuda").reshape(1, 32, 32))
+    plain, got = (capi.matmul_bfp(x, capi.ROW_MAJOR, words, BFP8, 1, 1, m, 32, 32, activation=act, out_dtype=torch.float32).reshape(m, 32).double()
+                  for act in (capi.ACT_NONE, capi.ACT_GELU))
+    want = 0.5 * plain * torch.special.erfc(-plain / 2.0 ** 0.5)
+    assert bool(((got - want).abs() <= 2.0 ** -21 * plain.abs()).all())
+
+
 def check_on_device(c, a, w, k):
     """The fp32 accumulation bound (2 k 2^-24 of the terms) on an fp32 result, evaluated in float64 on the GPU."""
     ref, terms = a.double() @ w.double(), a.double().abs() @ w.double().abs()
