@@ -192,7 +192,8 @@ TTMI_API int ttmi_matmul_bfp_ab(const uint32_t *a, int a_fmt, const uint32_t *b,
 
 /* Which kernel a block-float GEMM of this shape and these dtypes goes to, for whoever reads a profiler trace (no counterpart
  * in the reference, whose program factories log their choice; needs no GPU):
- *   out[0]  1 = 64-column streaming kernel, 2 = 128-column streaming kernel, 3 = fused tiled kernels, 4 = expansion + bf16 GEMM
+ *   out[0]  1 = 64-column streaming kernel, 2 = 128-column streaming kernel, 3 = fused tiled kernels, 4 = expansion + bf16 GEMM,
+ *          5 = expansion to bf16 tiles + the GEMM of ttmi_matmul_bf16
  *   out[1]  k ranges per output (workgroups that share an output), streaming kernels only, else 0
  *   out[2]  workgroups launched where the library knows nothing about workgroup placement
  *   out[3]  workgroups launched on a device whose consecutive workgroups go to 8 XCDs in turn (MI355X) */

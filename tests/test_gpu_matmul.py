@@ -911,3 +911,50 @@ def test_block_float_activations_where_no_kernel_takes_them():
     assert L.ttmi_matmul_bfp_ab(one, BFP4, one, BFP8, 1, 1, 32, 4096, 4096, None, 0, one, capi.TILE, capi.BFLOAT16, None, 0, None) == 3
     assert L.ttmi_matmul_bfp_ab(one, capi.BFLOAT16, one, BFP8, 1, 1, 32, 4096, 4096, None, 0, one, capi.TILE, capi.BFLOAT16, None, 0, None) == 1
     assert L.ttmi_matmul_bfp_ab(one, BFP8, one, BFP8, 1, 1, 40, 4096, 4096, None, 0, one, capi.ROW_MAJOR, capi.BFLOAT16, None, 0, None) == 1
+
+
+@pytest.mark.parametrize("block", [64, 128])
+@pytest.mark.parametrize("fmt", [BFP8, BFP4])
+@pytest.mark.parametrize("batch,b_batch,m,k,n", [(1, 1, 1, 96, 32), (2, 2, 130, 128, 160), (3, 1, 160, 1056, 288)])
+def test_weights_expanded_to_bf16_tiles(oracle, batch, b_batch, m, k, n, fmt, block, knobs):
+    """Block-float weights expanded to bf16 tiles for the kernel of two bf16 operands, against the expanding GEMM: the same
+    products, so only the order of the fp32 sums may differ (2 k 2^-24 of the terms each), also for rows at the ends of the
+    exponent range (E = 0, 254, 255: the same outputs are non-finite); every output form."""
+    rng = np.random.default_rng(540 + k)
+    w_bits = 7 if fmt == BFP8 else 3
+    exps = rng.integers(118, 131, size=(b_batch, k, n // 16)).astype(np.uint8)
+    codes = rng.integers(0, 1 << (w_bits + 1), size=(b_batch, k, n)).astype(np.uint8)
+    a = rng.standard_normal((batch, m, k)).astype(np.float32)
+    exps[:, 5], a[..., 5] = 0, a[..., 5] * 2.0 ** 124
+    exps[:, 77], a[..., 77] = 254, a[..., 77] * 2.0 ** -125
+    codes[:, 77, 16:] &= ~np.uint8((1 << w_bits) - 2)                   # mantissas of 0 and 1 stay finite there
+    exps[:, 90, 1] = 255
+    a_bits = workloads.f32_to_bf16_bits_rne(a)
+    a_dev = bf16_dev(a_bits).reshape(batch, m, k)
+    words = torch.from_numpy(np.concatenate([assemble_tiles(fmt, e, c).reshape(-1) for e, c in zip(exps, codes)]).view(np.int32)).cuda()
+    bias = bf16_dev(workloads.f32_to_bf16_bits_rne(workloads.normal_tensor((n,), seed=541)))
+    call = lambda a=a_dev, layout=capi.ROW_MAJOR, **more: capi.matmul_bfp(a, layout, words, fmt, batch, b_batch, m, k, n, bias=bias, **more)
+    knobs("kernel", "expanded")
+    want = call(out_dtype=torch.float32).cpu().numpy().astype(np.float64)
+    knobs("kernel", "bf16 in place")
+    knobs("block", block)
+    got_dev = call(out_dtype=torch.float32)
+    got = got_dev.cpu().numpy().astype(np.float64)
+    ok = np.isfinite(want)
+    assert np.array_equal(ok, np.isfinite(got)) and ok.any() and not ok[..., 16:32].any() and (n < 64 or ok[..., 32:].all())
+    mant = (codes & ((1 << w_bits) - 1)).astype(np.float64)
+    e_eff = np.minimum(np.maximum(np.repeat(exps, 16, axis=2).astype(np.int64), 1), 254)
+    terms = np.abs(workloads.bf16_bits_to_f32(a_bits).reshape(batch, m, k)).astype(np.float64) @ (mant * np.exp2((e_eff - 127 - (w_bits - 1)).astype(np.float64))) + 4.0
+    assert np.all(np.abs(got[ok] - want[ok]) <= (4.0 * k * 2.0 ** -24 * terms)[ok])
+    rounded = got_dev.bfloat16()
+    same = lambda c: torch.equal(torch.nan_to_num(c, 1.0, 2.0, 3.0), torch.nan_to_num(rounded, 1.0, 2.0, 3.0))
+    assert same(call())
+    assert torch.equal(call(activation=capi.ACT_RELU)[got_dev.isfinite()], torch.relu(rounded)[got_dev.isfinite()])
+    if m % 32 == 0:
+        a_tiles = capi.tilize(a_dev)
+        tiles = call(a_tiles, capi.TILE, c_layout=capi.TILE)
+        assert same(capi.untilize(tiles, (batch, m, n)))
+        packed = call(a_tiles, capi.TILE, c_layout=capi.TILE, out_bfp=fmt)
+        host = oracle.pack_fp32_vec_as_bfp_tiles(fmt, tiles.float().cpu().numpy().reshape(-1), False)
+        finite = np.isfinite(tiles.float().cpu().numpy().reshape(-1, 1024)).all(axis=1)          # tiles without the poisoned columns
+        assert np.array_equal(packed.cpu().numpy().view(np.uint32).reshape(len(finite), -1)[finite], host.reshape(len(finite), -1)[finite])

@@ -1139,7 +1139,7 @@ int matmul_bfp_wide(const MatmulArgs &x, hipStream_t st) { return launch_streami
 // [18176, 4544] BFP8_B 58.1 against 54.0, [4096, 4096] BFP8_B 17.6 against 15.6, [14336, 4096] BFP4_B 37.0 against 30.3).  Taller activations are MFMA-bound: the fused tiled kernels up to 511 rows, and from 512 rows
 // on (two or more 256-row blocks share every weight) the weights are expanded to bf16 once and a plain bf16 GEMM follows.
 // The test entry point can force a kernel (TTMI_KNOB_MATMUL_KERNEL).
-enum class Kernel { Stream = 1, Wide = 2, Tile = 3, Expanded = 4 };
+enum class Kernel { Stream = 1, Wide = 2, Tile = 3, Expanded = 4, Direct = 5 };
 static double streamed_estimate(uint32_t batch, uint32_t m, uint32_t k, uint32_t n, int b_fmt) {
     const double weights = (double)k * n * (b_fmt == TTMI_BFLOAT8_B ? 1.0625 : 0.8);     // BFLOAT4_B: half the bytes, the same instructions
     const double sets = (double)batch * (((m + 31) / 32 + 1) / 2);
@@ -1151,7 +1151,7 @@ static double tiled_estimate(uint32_t batch, uint32_t m, uint32_t k, uint32_t n)
 }
 static Kernel choose_kernel(uint32_t batch, uint32_t m, uint32_t k, uint32_t n, int b_fmt, bool c_bfp) {
     uint32_t forced;
-    if (knob(TTMI_KNOB_MATMUL_KERNEL, &forced) && forced >= 1 && forced <= 4) return (Kernel)forced;
+    if (knob(TTMI_KNOB_MATMUL_KERNEL, &forced) && forced >= 1 && forced <= 5) return (Kernel)forced;
     if (m >= 128) {
         // Tall activations are MFMA-bound when the output has enough blocks for the chip: a 128 x 256 or 256 x 256 block per
         // workgroup takes about 0.75 us per k-tile, and a GEMM with few columns leaves most CUs without one.  Streaming the
@@ -1190,30 +1190,38 @@ static Kernel choose_kernel(uint32_t batch, uint32_t m, uint32_t k, uint32_t n, 
 // matmul_workspace_bytes, has no room for the partial sums), which is what outputs of few blocks and last rounds on a part
 // of the chip need.  Measured, same box: [1000, 14336] x [14336, 4096] BFLOAT4_B, 64 blocks, 152 us in four k ranges against
 // 205 streamed; [200, 4096] x [4096, 14336] and [300, 16384] x [16384, 16384] are better streamed (63 us, 310 us), as estimated.
-static Kernel choose_kernel_own_scratch(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, int b_fmt, bool c_bfp) {
+// And the weights can be expanded to bf16 tiles for the kernel that takes two bf16 operands, whose smaller blocks fill the chip
+// where 256 x 256 blocks do not and the rows are too many to stream for.  Measured, streamed / cut into k ranges / that: 8 x
+// [384, 4096] x [4096, 1024] 58 / 53 / 44 us, [1024, 4096] x [4096, 4096] 57 / 59 / 54; not where the rows are fewer ([512,
+// 4096] x [4096, 1024] 16 / 29 / 30, [416, 4096] x [4096, 4096] 34 / 48 / 46) or the weights are many ([2048, 4544] x [4544,
+// 4672] 172 / 104 / 115).
+struct Choice { Kernel kernel; double us; };
+static Choice choose_kernel_own_scratch(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, int b_fmt, bool c_bfp) {
     const Kernel kernel = choose_kernel(batch, m, k, n, b_fmt, c_bfp);
+    const double bytes_per_weight = b_fmt == TTMI_BFLOAT8_B ? 1.0625 : 0.5625;
+    const double expanded = matmul_expanded_estimate(batch, b_batch, m, k, n, bytes_per_weight);
+    const Choice as_ever{kernel, kernel == Kernel::Expanded ? expanded : kernel == Kernel::Tile ? tiled_estimate(batch, m, k, n) : streamed_estimate(batch, m, k, n, b_fmt)};
     uint32_t forced;
-    if (m < 128 || kernel == Kernel::Expanded || knob(TTMI_KNOB_MATMUL_KERNEL, &forced)) return kernel;
-    const double now = kernel == Kernel::Tile ? tiled_estimate(batch, m, k, n) : streamed_estimate(batch, m, k, n, b_fmt);
-    const double expanded = matmul_expanded_estimate(batch, b_batch, m, k, n, b_fmt == TTMI_BFLOAT8_B ? 1.0625 : 0.5625);
-    return expanded < 0.95 * now ? Kernel::Expanded : kernel;
+    if (m < 128 || ((uint64_t)m + 31) / 32 * 64 * k > 0xffffffffull || knob(TTMI_KNOB_MATMUL_KERNEL, &forced)) return as_ever;     // (A of 4 GiB: validate_expanded)
+    Choice best = as_ever;
+    if (expanded < 0.95 * best.us) best = {Kernel::Expanded, expanded};
+    const double direct = matmul_direct_estimate(batch, b_batch, m, k, n, bytes_per_weight);
+    if (direct < 0.9 * best.us) best = {Kernel::Direct, direct};
+    return best;
 }
 
 // Slices that share their weights are one GEMM of all their rows: [batch, m, k] lies in memory as [1, batch m, k] does, dense
 // or in whole tiles (TILE layouts have m % 32 == 0), and blocks of rows need not end with a slice.  Taken where the rows
-// together go to the expanding GEMM and it is the better one: 8 x [384, 1024] x [1024, 4096] 39 us against 67 slice by slice
-// (tiled).  Not for streamed shapes, whose slices share the weights through the caches: 2 x [32, 4096] x [4096, 4096] 13.6
-// against 10.2 us as they are.
+// together go to the expanding GEMM (or the one with smaller blocks) and that is the better one: 8 x [384, 1024] x [1024,
+// 4096] 39 us against 67 slice by slice (tiled).  Not for streamed shapes, whose slices share the weights through the caches:
+// 2 x [32, 4096] x [4096, 4096] 13.6 against 10.2 us as they are.
 static bool fold_batch(const MatmulArgs &x, bool c_bfp) {
     const uint64_t rows = (uint64_t)x.batch * x.m;
     uint32_t forced;
     if (x.b_batch != 1 || x.batch == 1 || rows * x.k * 2 > 0xffffffffull || rows > 0x7fffff00ull || knob(TTMI_KNOB_MATMUL_KERNEL, &forced)) return false;
-    if (choose_kernel_own_scratch(1, 1, (uint32_t)rows, x.k, x.n, x.b_fmt, c_bfp) != Kernel::Expanded) return false;
-    const double bytes = x.b_fmt == TTMI_BFLOAT8_B ? 1.0625 : 0.5625;
-    const Kernel as_is = choose_kernel_own_scratch(x.batch, 1, x.m, x.k, x.n, x.b_fmt, c_bfp);
-    const double slices = as_is == Kernel::Expanded ? matmul_expanded_estimate(x.batch, 1, x.m, x.k, x.n, bytes)
-                        : as_is == Kernel::Tile ? tiled_estimate(x.batch, x.m, x.k, x.n) : streamed_estimate(x.batch, x.m, x.k, x.n, x.b_fmt);
-    return matmul_expanded_estimate(1, 1, (uint32_t)rows, x.k, x.n, bytes) < slices;
+    const Choice folded = choose_kernel_own_scratch(1, 1, (uint32_t)rows, x.k, x.n, x.b_fmt, c_bfp);
+    if (folded.kernel != Kernel::Expanded && folded.kernel != Kernel::Direct) return false;
+    return folded.us < choose_kernel_own_scratch(x.batch, 1, x.m, x.k, x.n, x.b_fmt, c_bfp).us;
 }
 
 size_t matmul_gated_workspace_bytes(uint32_t batch, uint32_t m, uint32_t k, uint32_t n) {
@@ -1240,7 +1248,7 @@ size_t matmul_workspace_bytes(uint32_t batch, uint32_t m, uint32_t k, uint32_t n
 void matmul_plan(uint32_t batch, uint32_t m, uint32_t k, uint32_t n, int b_fmt, bool a_or_c_bfp, uint32_t out[4]) {
     out[0] = out[1] = out[2] = out[3] = 0;
     if (!batch || !m || !k || !n) return;
-    const Kernel kernel = choose_kernel_own_scratch(batch, batch, m, k, n, b_fmt, a_or_c_bfp);
+    const Kernel kernel = choose_kernel_own_scratch(batch, batch, m, k, n, b_fmt, a_or_c_bfp).kernel;
     out[0] = (uint32_t)kernel;
     if (kernel != Kernel::Wide && kernel != Kernel::Stream) return;
     const bool wide = kernel == Kernel::Wide;
@@ -1267,12 +1275,13 @@ int matmul_bfp(const MatmulArgs &asked, hipStream_t st) {
     // (the workspace query answers for the slices as they are, so a caller's workspace serves those)
     const bool own_scratch = !x.workspace && !x.no_alloc;
     if (own_scratch && !a8 && fold_batch(x, c_bfp)) { x.m *= x.batch; x.batch = 1; }
-    const Kernel kernel = own_scratch ? choose_kernel_own_scratch(x.batch, x.b_batch, x.m, x.k, x.n, x.b_fmt, c_bfp || a8)
+    const Kernel kernel = own_scratch ? choose_kernel_own_scratch(x.batch, x.b_batch, x.m, x.k, x.n, x.b_fmt, c_bfp || a8).kernel
                                       : choose_kernel(x.batch, x.m, x.k, x.n, x.b_fmt, c_bfp || a8);
     if (a8 && !matmul_takes_bfp_activations(x.batch, x.m, x.k, x.n, x.b_fmt))
         return fail(TTMI_ERR_UNSUPPORTED, "matmul: block-float activations are taken by the one-band streaming kernel only, which this shape does "
                     "not go to (ttmi_matmul_bfp_ab_supported): expand them with ttmi_typecast_tiles first");
     switch (kernel) {
+        case Kernel::Direct: return matmul_bf16_direct(x, st);
         case Kernel::Expanded: return matmul_bfp_expanded(x, st);
         case Kernel::Tile: return matmul_bfp_tiled(x, st);
         case Kernel::Wide: return matmul_bfp_wide(x, st);

@@ -3,7 +3,8 @@
 // What it is for: batched products whose operands are both activations (scores and context of an attention layer: every
 // head brings weights of its own, used once), where a re-layout pass costs as much as the product, and outputs too small
 // or too narrow for the 256 x 256 blocks of matmul_expanded_kernel.  Those products move more bytes than they have work
-// for the matrix cores (8 x 16 heads of [384, 64] x [64, 384]: 50 MB, 2.4 GFLOP), so HBM bounds them.
+// for the matrix cores (8 x 16 heads of [384, 64] x [64, 384]: 50 MB, 2.4 GFLOP), so HBM bounds them.  Block-float weights come
+// here, expanded to bf16 tiles by expand_tiles_kernel, where blocks of 64 or 128 fill the chip and 256 x 256 ones do not.
 //
 //   block      32 RB WR rows x 32 CB WC columns of C per workgroup of four wavefronts (WR x WC of them)
 //   staging    one k tile row (32 k values) per step, whole tiles of A and B through a ring of LDS stages filled by direct
@@ -41,6 +42,7 @@ struct DirectDev {
     uint32_t kt, nt, mt, tiles_m, tiles_n, blocks, per_xcd;
     int a_tiled, c_tiled, c_f32;
     int c_bfp;               // 0, or the mantissa bits (7 | 3) of a block-float output in TILE layout
+    float unscale;           // common factor of the products: 1, or Wfmt::unscale for expanded block floats
 };
 
 // LDS reads are written as inline assembly: the compiler orders every transposing read behind ALL outstanding direct-to-LDS
@@ -187,11 +189,11 @@ __global__ __launch_bounds__(256, 2) void matmul_direct_kernel(const DirectDev p
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     uint2 bias4 = make_uint2(0u, 0u);
-                    if (p.bias) bias4 = *reinterpret_cast<const uint2 *>(p.bias + col_tile * 32 + f * 16 + h * 8 + kh * 4);
+                    if (p.bias) __builtin_memcpy(&bias4, p.bias + col_tile * 32 + f * 16 + h * 8 + kh * 4, 8);      // a bias need not be aligned
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const uint32_t w = i < 2 ? bias4.x : bias4.y;
-                        v[h * 4 + i] = apply_activation<ACT>(acc[rb][cb][(2 * f + h) * 4 + i] + __uint_as_float((i & 1) ? w & 0xffff0000u : w << 16));
+                        v[h * 4 + i] = apply_activation<ACT>(acc[rb][cb][(2 * f + h) * 4 + i] * p.unscale + __uint_as_float((i & 1) ? w & 0xffff0000u : w << 16));
                     }
                 }
                 if (p.c_f32) {
@@ -244,6 +246,46 @@ __global__ __launch_bounds__(256, 2) void matmul_direct_kernel(const DirectDev p
     }
 }
 
+// Packed tiles -> bf16 tiles in the same element order, for a GEMM of block-float weights on the kernel above: 8 elements per lane
+// and piece, four pieces in flight.  HBM-bound.  The values carry the common factor of Wfmt::unscale, and the ends of the
+// exponent range come out as in expand_kernel.
+template <int W>
+__global__ __launch_bounds__(256) void expand_tiles_kernel(const uint8_t *__restrict__ b, u32x4 *__restrict__ out, uint64_t pieces) {
+    constexpr int PIECES = 4;
+    const uint64_t first = (uint64_t)blockIdx.x * (256 * PIECES) + threadIdx.x;
+    uint32_t words[PIECES][2], exps[PIECES];
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+        const uint64_t at = min(first + j * 256, pieces - 1);
+        const uint32_t piece = (uint32_t)at & 127;                       // of the tile's 128
+        const uint8_t *tile = b + (at >> 7) * Wfmt<W>::tile_bytes;
+        exps[j] = tile[piece >> 1];
+        if (W == 7) {
+            const uint2 v = *reinterpret_cast<const uint2 *>(tile + 64 + piece * 8);
+            words[j][0] = v.x; words[j][1] = v.y;
+        } else {
+            words[j][0] = *reinterpret_cast<const uint32_t *>(tile + 64 + piece * 4);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+        const float scale = row_scale(exps[j]);
+        u32x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            uint32_t bits[2];
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const int e = 2 * i + h;
+                const uint32_t code = W == 7 ? words[j][e >> 2] >> (8 * (e & 3)) : words[j][0] >> (4 * e);
+                bits[h] = __float_as_uint((float)(code & ((1u << W) - 1)) * scale) | ((code >> W) & 1u) << 31;      // at most 7 significant bits
+            }
+            v[i] = (bits[1] & 0xffff0000u) | bits[0] >> 16;
+        }
+        if (first + j * 256 < pieces) out[first + j * 256] = v;
+    }
+}
+
 namespace {
 template <int WR, int WC, int RB, int CB, int STAGES> int launch_direct(DirectDev p, const MatmulArgs &x, hipStream_t st) {
     p.tiles_m = (p.mt + WR * RB - 1) / (WR * RB);
@@ -264,18 +306,27 @@ template <int WR, int WC, int RB, int CB, int STAGES> int launch_direct(DirectDe
 }  // namespace
 
 // Rows and columns of the block a shape goes to, 0 for the re-layout and 256 x 256 blocks.  Estimates from these
-// measurements (us, one MI355X; 64 / 128 / 256 blocks): a k tile row takes a 128 x 128 block 0.27 to 0.31 us and a CU gains
-// nothing from a second block ([512, 2048] x [2048, 2048], a quarter of the chip: 22 us; [2048, 4096] x [4096, 4096], two
-// per CU: 68); a 64 x 64 block 0.165 us alone and 0.143 us as one of many ([256, 8192] x [8192, 1024] 43 / 74 / 144, [4096,
-// 4096] x [4096, 4096] 293 / 159 / 130); a 256 x 256 block 0.72 us behind a pass over the weights and a second launch.
-uint32_t bf16_direct_block(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n) {
+// measurements (us, one MI355X; 64 / 128 / 256 blocks): a k tile row takes a 128 x 128 block 0.31 us alone on its CU and 0.27
+// as one of several ([512, 2048] x [2048, 2048], a quarter of the chip: 22 us; [2048, 4096] x [4096, 4096], two per CU: 68); a
+// 64 x 64 block 0.165 us alone and 0.143 us as one of many, 0.1 where the weights are few columns, which every L2 keeps
+// ([256, 8192] x [8192, 1024] 43 / 74 / 144, [4096, 4096] x [4096, 4096] 293 / 159 / 130, [3072, 4096] x [4096, 1024], block-float
+// weights, 44 / 47 / 53); a 256 x 256 block 0.72 us behind a pass over the weights and a second launch.
+static double direct_us(uint32_t batch, uint32_t m, uint32_t k, uint32_t n, uint32_t *block) {
     const double steps = k / 32;
     auto blocks = [&](uint32_t edge) { return (double)batch * ((m + edge - 1) / edge) * ((n + edge - 1) / edge) / 256.0; };
-    const double at64 = steps * std::max(0.165, blocks(64) * 0.143);
-    const double at128 = steps * std::ceil(blocks(128)) * 0.285;
-    const double at256 = 8.0 + (double)b_batch * k * n * 4.0 / 5.0e6 + steps * std::ceil(blocks(256)) * 0.72;
-    if (at256 < std::min(at64, at128)) return 0;
-    return at64 < at128 ? 64 : 128;
+    const double at64 = steps * std::max(0.165, blocks(64) * (n <= 1024 ? 0.1 : 0.143)),
+                 at128 = steps * (blocks(128) <= 1.0 ? 0.31 : std::ceil(blocks(128)) * 0.27);
+    if (block) *block = at64 < at128 ? 64 : 128;
+    return std::min(at64, at128);
+}
+uint32_t bf16_direct_block(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n) {
+    uint32_t block;
+    const double direct = direct_us(batch, m, k, n, &block), blocks = (double)batch * ((m + 255) / 256) * ((n + 255) / 256);
+    return 8.0 + (double)b_batch * k * n * 4.0 / 5.0e6 + (k / 32) * std::ceil(blocks / 256.0) * 0.72 < direct ? 0 : block;
+}
+// With a pass in front that expands block-float weights to bf16 tiles.
+double matmul_direct_estimate(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, double bytes_per_weight) {
+    return 5.0 + (double)b_batch * k * n * (bytes_per_weight + 2.0) / 4.0e6 + direct_us(batch, m, k, n, nullptr);
 }
 
 int matmul_bf16_direct(const MatmulArgs &x, hipStream_t st) {
@@ -285,8 +336,24 @@ int matmul_bf16_direct(const MatmulArgs &x, hipStream_t st) {
     p.kt = x.k / 32; p.nt = x.n / 32; p.mt = (x.m + 31) / 32;
     p.a_tiled = x.a_layout == TTMI_TILE; p.c_tiled = x.c_layout == TTMI_TILE; p.c_f32 = x.c_dtype == TTMI_FLOAT32;
     p.c_bfp = x.c_dtype == TTMI_BFLOAT8_B ? 7 : x.c_dtype == TTMI_BFLOAT4_B ? 3 : 0;
-    uint32_t block = bf16_direct_block(x.batch, x.b_batch, x.m, x.k, x.n);
-    block = knob_or(TTMI_KNOB_MATMUL_BLOCK, block ? block : 128);
+    p.unscale = 1.0f;
+    if (x.b_fmt != TTMI_BFLOAT16) {                             // scratch of the library's own, which callers without it do not come here for
+        const uint64_t pieces = (uint64_t)x.b_batch * p.kt * p.nt * 128, blocks = (pieces + 1023) / 1024;
+        if (blocks > 0x7fffffffull) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: problem too large for one launch");
+        void *dense;
+        bool fresh;
+        if (int rc = scratch_get(SCRATCH_EXPANDED, st, (size_t)pieces * 16, &dense, &fresh)) return rc;
+        if (x.b_fmt == TTMI_BFLOAT8_B)
+            hipLaunchKernelGGL((expand_tiles_kernel<7>), dim3((uint32_t)blocks), dim3(256), 0, st, p.b, (u32x4 *)dense, pieces);
+        else
+            hipLaunchKernelGGL((expand_tiles_kernel<3>), dim3((uint32_t)blocks), dim3(256), 0, st, p.b, (u32x4 *)dense, pieces);
+        if (int rc = check_launch("expand_tiles_kernel")) return rc;
+        p.b = (const uint8_t *)dense;
+        p.unscale = x.b_fmt == TTMI_BFLOAT8_B ? Wfmt<7>::unscale : Wfmt<3>::unscale;
+    }
+    uint32_t block;
+    direct_us(x.batch, x.m, x.k, x.n, &block);
+    block = knob_or(TTMI_KNOB_MATMUL_BLOCK, block);
     return block == 128 ? launch_direct<2, 2, 2, 2, 3>(p, x, st) : launch_direct<2, 2, 1, 1, 4>(p, x, st);
 }
 

@@ -29,7 +29,7 @@ bool error_word_if_exists(uint32_t **device_ptr, volatile uint32_t **host_ptr); 
 // Knobs of the test entry point ttmi_test_set_knob(which, value, set), which only the test build of the library has
 // (-DTTMI_TEST_HOOKS: libttmi_test.so); in the product library every knob reads as unset.
 enum {
-    TTMI_KNOB_MATMUL_KERNEL = 0,      // 1 stream (64 columns), 2 wide (128 columns), 3 tiled, 4 expanded; bf16 weights: 4 expanded, 5 in place
+    TTMI_KNOB_MATMUL_KERNEL = 0,      // 1 stream (64 columns), 2 wide (128 columns), 3 tiled, 4 expanded, 5 expanded to bf16 tiles; bf16 weights: 4 expanded, 5 in place
     TTMI_KNOB_MATMUL_WORKGROUPS = 1,  // workgroups the streaming kernels aim for
     TTMI_KNOB_MATMUL_BLOCK = 2,       // block form of the tiled kernels: 256, 128 (eight wavefronts), 4 (128 rows, four wavefronts), 384; bf16 weights in place: 128, 64
     TTMI_KNOB_SPIN_LIMIT = 3,         // polls before a bounded wait gives up
@@ -93,8 +93,9 @@ int matmul_bfp_gated(const MatmulArgs &args, hipStream_t st);   // args.b2 set
 int matmul_bf16(const MatmulArgs &args, hipStream_t st);        // args.b: bf16 tiles, args.b_fmt = TTMI_BFLOAT16
 int matmul_bfp_tiled(const MatmulArgs &args, hipStream_t st);
 int matmul_bfp_expanded(const MatmulArgs &args, hipStream_t st);   // expand the weights to bf16 once, then a bf16 GEMM
-int matmul_bf16_direct(const MatmulArgs &args, hipStream_t st);    // bf16 weights read as they lie, no pass over them first
+int matmul_bf16_direct(const MatmulArgs &args, hipStream_t st);    // bf16 weights read as they lie; block-float ones expanded to bf16 tiles first, in scratch of the library's own
 uint32_t bf16_direct_block(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n);    // the block edge a shape gets there, 0: not for it
+double matmul_direct_estimate(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, double bytes_per_weight);    // us, behind a pass that expands the weights
 int validate_expanded(const MatmulArgs &args);
 double matmul_expanded_estimate(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, double bytes_per_weight);   // us, k ranges cut where that helps
 size_t matmul_expanded_workspace_bytes(uint32_t b_batch, uint32_t k, uint32_t n);
