@@ -740,9 +740,9 @@ def test_bf16_weights(batch, b_batch, m, k, n):
 @pytest.mark.parametrize("kernel", ["stream", "wide", "tile", "expanded"])
 def test_gelu_over_its_range(kernel, knobs):
     """GELU of the values that a product with the identity gives in fp32 (the same call without activation says which: the streaming
-    kernels' sums pass through neighbours of the weights, so they need not be the inputs bit for bit), where its two forms of
-    erf meet (|x| = sqrt(2)), where erf reaches 1 and far beyond.  Bound: erf to 7.1e-8, its argument to 2^-24 (x d erf / dx <= 0.5 in relative terms), the sum
-    1 + erf and two products to 2^-24 each: less than 2^-21 |x| in all."""
+    kernels' sums pass through neighbours of the weights, so they need not be the inputs bit for bit), where the fit of the tail
+    ends (|x| = 6), where the tail vanishes and far beyond.  Bound: the tail 2^-L to 4.7e-10 + ln 2 max(L 2^-L) (11 roundings of L
+    at most) 2^-24, one product and sum to 2^-24: less than 2^-21 |x| in all."""
     knobs("kernel", kernel)
     x = torch.cat([torch.linspace(-9, 9, 3000), torch.linspace(-1.43, -1.40, 500), torch.linspace(1.40, 1.43, 500),
                    torch.tensor([0.0, -0.0, 1e-30, -1e-30, 40.0, -40.0, 1e4, -1e4])])
