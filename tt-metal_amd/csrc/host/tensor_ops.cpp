@@ -12,7 +12,6 @@
 #include <functional>
 #include <mutex>
 #include <stdexcept>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -166,7 +165,7 @@ bool through_slots(void *host, bool to_device, uint32_t batch, uint32_t h, size_
     int started = 1;
     try {
         for (; started < SLOT_WORKERS; ++started) threads.emplace_back(work, started);
-    } catch (const std::system_error &) {                       // no more threads to be had: their share is done below
+    } catch (...) {                                             // no more threads (or memory) to be had: their share is done below
     }
     work(0);
     for (int w = started; w < SLOT_WORKERS; ++w) work(w);
