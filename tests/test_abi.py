@@ -102,6 +102,35 @@ def test_argument_validation_returns_errors_without_launching():
         assert b"weight dtype" in L.ttmi_last_error()
 
 
+@pytest.mark.parametrize("m,k,n", [(32, 64, 64), (32, 4096, 4096), (96, 4544, 4672), (200, 4096, 14336), (384, 1024, 1024), (1024, 4096, 4096), (2048, 4544, 18176)])
+@pytest.mark.parametrize("batch,b_batch", [(1, 1), (4, 1), (4, 4)])
+def test_misaligned_operands_are_refused_by_every_gemm(m, k, n, batch, b_batch):
+    """Whichever kernel a shape goes to (all of them are among these), with the library's scratch, a workspace or none: a, b, b_up and
+    c move in pieces of up to 16 bytes, so an address that is no multiple of 16 is an error before anything else happens.  A
+    bias may lie anywhere."""
+    from ttmi import capi
+
+    if not os.path.exists(capi.LIB_PATH):
+        pytest.skip("libttmi.so not built")
+    L = capi.lib()
+    sizes = (batch, b_batch, m, k, n)
+    calls = {
+        "bfp": lambda a, b, up, c: L.ttmi_matmul_bfp(a, 0, b, 3, *sizes, None, 0, c, 0, 0, None, 0, None),
+        "bfp, workspace": lambda a, b, up, c: L.ttmi_matmul_bfp(a, 0, b, 4, *sizes, None, 0, c, 0, 1, ctypes.c_void_p(4096), 1 << 30, None),
+        "static": lambda a, b, up, c: L.ttmi_matmul_bfp_static(a, 0, b, 3, *sizes, None, 0, c, 0, 0, None),
+        "bf16": lambda a, b, up, c: L.ttmi_matmul_bf16(a, 0, b, *sizes, None, 0, c, 0, 0, None, 0, None),
+        "gated": lambda a, b, up, c: L.ttmi_matmul_bfp_gated(a, 0, b, up, 3, *sizes, None, 0, c, 0, 0, None, 0, None),
+    }
+    for name, call in calls.items():
+        for which in range(4):
+            if which == 2 and name != "gated":
+                continue
+            for off in (2, 8):
+                operands = [ctypes.c_void_p(4096 + (off if i == which else 0)) for i in range(4)]
+                assert call(*operands) == 1, (name, which, off)
+                assert b"16-byte aligned" in L.ttmi_last_error(), (name, which, off, L.ttmi_last_error())
+
+
 def test_missing_library_fails_loudly(monkeypatch):
     from ttmi import capi
 

@@ -1062,8 +1062,6 @@ static int launch_streaming(const MatmulArgs &x, hipStream_t st, bool wide) {
     p.c_f32 = x.c_dtype == TTMI_FLOAT32;
     p.c_bfp = x.c_dtype == TTMI_BFLOAT8_B ? 7 : x.c_dtype == TTMI_BFLOAT4_B ? 3 : 0;
     if (p.c_bfp && !(wide && p.c_tiled)) return fail(TTMI_ERR_UNSUPPORTED, "matmul: this kernel writes no block-float output");
-    if ((reinterpret_cast<uintptr_t>(x.a) | reinterpret_cast<uintptr_t>(x.b) | reinterpret_cast<uintptr_t>(x.b2) | reinterpret_cast<uintptr_t>(x.c)) & 15u)
-        return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: a, b and c must be 16-byte aligned");
     if (d.units > 0x7fffffffull || d.groups * d.split > 0x7fffffffull) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: problem too large for one launch");
     const bool bands2 = two_bands(x.m, wide, gated);
     const size_t need = slot_bytes_needed(d, wide, gated || bands2);

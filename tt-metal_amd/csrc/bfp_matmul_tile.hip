@@ -756,8 +756,6 @@ int matmul_bfp_tiled(const MatmulArgs &x, hipStream_t st) {
         if (blocks_tall > 0x7fffffffull) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: problem too large for one launch");
         if ((uint64_t)x.m * x.k * 2 > 0xffffffffull || (uint64_t)((x.m + 31) / 32) * p.kt * 2048 > 0xffffffffull)
             return fail(TTMI_ERR_UNSUPPORTED, "matmul: one batch slice of A exceeds 4 GiB");
-        if ((reinterpret_cast<uintptr_t>(x.a) | reinterpret_cast<uintptr_t>(x.b) | reinterpret_cast<uintptr_t>(x.c)) & 15u)
-            return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: a, b and c must be 16-byte aligned");
         if (x.b_fmt == TTMI_BFLOAT8_B) launch_tall_act<7, TALL_WAVES>(p, x.activation, (uint32_t)blocks_tall, st);
         else launch_tall_act<3, TALL_WAVES>(p, x.activation, (uint32_t)blocks_tall, st);
         return check_launch("matmul_tall_kernel");
@@ -772,8 +770,6 @@ int matmul_bfp_tiled(const MatmulArgs &x, hipStream_t st) {
     if (blocks > 0x7fffffffull) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: problem too large for one launch");
     if ((uint64_t)x.m * x.k * 2 > 0xffffffffull || (uint64_t)((x.m + 31) / 32) * p.kt * 2048 > 0xffffffffull)
         return fail(TTMI_ERR_UNSUPPORTED, "matmul: one batch slice of A exceeds 4 GiB");
-    if ((reinterpret_cast<uintptr_t>(x.a) | reinterpret_cast<uintptr_t>(x.b) | reinterpret_cast<uintptr_t>(x.c)) & 15u)
-        return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: a, b and c must be 16-byte aligned");
     if (x.b_fmt == TTMI_BFLOAT8_B) {
         if (use_256) launch_tile8_act<7, 4>(p, x.activation, (uint32_t)blocks, st);
         else if (four_waves) launch_tile_act<7, 4>(p, x.activation, (uint32_t)blocks, st);

@@ -42,6 +42,9 @@ int validate_matmul(const void *a, int a_layout, const uint32_t *b, int b_fmt, u
         return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: output dtype must be BFLOAT16, FLOAT32, BFLOAT8_B or BFLOAT4_B");
     if (is_bfp(c_dtype) && c_layout != TTMI_TILE) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: a block-float output needs TILE layout");
     if (activation < TTMI_ACT_NONE || activation > TTMI_ACT_SILU) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: unknown activation %d", activation);
+    // whichever kernel the shape goes to: all of them move a, b and c in pieces of up to 16 bytes
+    if ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c)) & 15u)
+        return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: a, b and c must be 16-byte aligned");
     return TTMI_OK;
 }
 
@@ -195,6 +198,7 @@ int ttmi_matmul_bfp_gated(const void *a, int a_layout, const uint32_t *b_gate, c
                           void *workspace, size_t workspace_bytes, void *stream) {
     if (int rc = validate_matmul(a, a_layout, b_gate, b_fmt, batch, b_batch, m, k, n, activation, c, c_layout, c_dtype)) return rc;
     if (!b_up) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: null pointer");
+    if (reinterpret_cast<uintptr_t>(b_up) & 15u) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: a, b and c must be 16-byte aligned");
     MatmulArgs args{a, a_layout, b_gate, b_fmt, batch, b_batch, m, k, n, bias, activation, c, c_layout, c_dtype, workspace, workspace_bytes};
     args.b2 = b_up;
     return matmul_bfp_gated(args, (hipStream_t)stream);
