@@ -140,3 +140,68 @@ def test_tall_kernel_mfma_writing_a_ring_register_in_flight_is_rejected(tmp_path
 
 def test_tall_kernel_without_inline_loads_is_reported(tmp_path):
     assert run_tall(tmp_path, "\tv_mfma_f32_32x32x16_bf16 v[2:17], v[34:37], v[82:85], v[2:17]\n") > 0
+
+
+# ---- the GEMM of two bf16 operands: LDS reads in flight behind the kernel's own partial lgkmcnt ----------------------------
+DIRECT_HEAD = "_ZN4ttmi20matmul_direct_kernelILi0ELi2ELi2ELi1ELi1ELi4EEEvNS_9DirectDevE:\n"
+
+
+def run_direct(tmp_path, body):
+    f = tmp_path / "d.s"
+    f.write_text(DIRECT_HEAD + body + TAIL)
+    return check_isa.check_lds_order(str(f))
+
+
+DIRECT_OK = (
+    ".LBB0_1:\n"
+    + asm("ds_read_b64_tr_b16 v[8:9], v1 offset:0") + asm("ds_read_b128 v[12:15], v2 offset:0")
+    + asm("ds_read_b64_tr_b16 v[10:11], v1 offset:1024") + asm("ds_read_b128 v[2:5], v2 offset:512")      # over its own address
+    + asm("s_waitcnt lgkmcnt(2)")
+    + "\tv_mfma_f32_32x32x16_bf16 v[20:35], v[8:9], v[12:15], v[20:35]\n"
+    + asm("s_waitcnt lgkmcnt(0)")
+    + "\tv_mfma_f32_32x32x16_bf16 v[20:35], v[10:11], v[2:5], v[20:35]\n"
+    + "\ts_cbranch_scc1 .LBB0_1\n"
+)
+
+
+def test_reads_behind_a_partial_wait_pass(tmp_path):
+    assert run_direct(tmp_path, DIRECT_OK) == 0
+    assert run_direct(tmp_path, "\ts_load_dwordx4 s[4:7], s[0:1], 0x0\n" + DIRECT_OK) == 0
+
+
+def test_a_wait_that_is_too_weak_is_reported(tmp_path, capsys):
+    assert run_direct(tmp_path, DIRECT_OK.replace("lgkmcnt(2)", "lgkmcnt(3)")) == 1
+    assert "[12, 13, 14, 15]" in capsys.readouterr().err
+    assert run_direct(tmp_path, DIRECT_OK.replace("lgkmcnt(0)", "vmcnt(0)")) > 0
+
+
+def test_a_younger_operation_of_the_compiler_counts_in_the_queue(tmp_path):
+    spill = DIRECT_OK.replace(asm("s_waitcnt lgkmcnt(2)"), "\tds_write_b32 v40, v41\n" + asm("s_waitcnt lgkmcnt(2)"))
+    assert run_direct(tmp_path, spill) == 0                        # the write is the youngest: one read more has landed, no less
+
+
+def test_a_copy_or_reuse_of_a_register_in_flight_is_reported(tmp_path):
+    copy = "\tv_mov_b32_e32 v50, v11\n"
+    assert run_direct(tmp_path, DIRECT_OK.replace(asm("s_waitcnt lgkmcnt(0)"), copy + asm("s_waitcnt lgkmcnt(0)"))) == 1
+    reuse = "\tds_read_b32 v10, v40\n"
+    assert run_direct(tmp_path, DIRECT_OK.replace(asm("s_waitcnt lgkmcnt(2)"), reuse + asm("s_waitcnt lgkmcnt(3)"))) == 1
+
+
+def test_a_read_in_flight_over_the_back_edge_or_at_the_end_is_reported(tmp_path):
+    open_end = DIRECT_OK.replace("\ts_cbranch_scc1 .LBB0_1\n", asm("ds_read_b64 v[60:61], v1") + "\ts_cbranch_scc1 .LBB0_1\n")
+    assert run_direct(tmp_path, open_end) == 1
+    back = DIRECT_OK.replace(".LBB0_1:\n", ".LBB0_1:\n\tv_mov_b32_e32 v50, v60\n").replace("\ts_cbranch_scc1 .LBB0_1\n", asm("ds_read_b64 v[60:61], v1") + "\ts_cbranch_scc1 .LBB0_1\n" + asm("s_waitcnt lgkmcnt(0)"))
+    assert run_direct(tmp_path, back) > 0
+
+
+def test_the_direct_kernel_without_inline_reads_is_reported(tmp_path):
+    assert run_direct(tmp_path, "\tv_mov_b32_e32 v1, v2\n") == 1
+
+
+def test_every_file_with_inline_lds_reads_is_checked_in_the_build():
+    import build
+
+    for src in build.SOURCES:
+        with open(os.path.join(build.CSRC, src)) as f:
+            text = f.read()
+        assert src in build.ISA_CHECKED or 'asm volatile("ds_read' not in text, src

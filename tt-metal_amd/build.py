@@ -25,7 +25,7 @@ LIB_TEST = os.path.join(LIB_DIR, "libttmi_test.so")
 HOOKED = ["host_state.hip", "bfp_matmul.hip", "bfp_matmul_tile.hip", "bfp_matmul_bf16.hip"]
 SOURCES = ["ttmi_capi.hip", "host_state.hip", "bfp_codec.hip", "bfp_matmul.hip", "bfp_matmul_tile.hip", "bfp_matmul_expanded.hip", "bfp_matmul_bf16.hip", "eltwise.hip"]
 # files whose device assembly is inspected before the object is built, and the check of check_isa.py that applies
-ISA_CHECKED = {"bfp_matmul.hip": "check", "bfp_matmul_tile.hip": "check_ring_operands"}
+ISA_CHECKED = {"bfp_matmul.hip": "check", "bfp_matmul_tile.hip": "check_ring_operands", "bfp_matmul_bf16.hip": "check_lds_order"}
 HEADERS = [os.path.join(CSRC, "ttmi_internal.h"), os.path.join(CSRC, "bfp_dequant.h"), os.path.join(ROOT, "include", "ttmi.h")]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

@@ -21,7 +21,8 @@ still in flight when the kernel ends.
     python tt-metal_amd/check_isa.py file.s
 
 A second, simpler check (check_ring_operands, `--ring-operands file.s`) covers the 384-row kernel of bfp_matmul_tile.hip,
-whose inline loads of A land in registers that the MFMAs read directly; it is described at the function.
+whose inline loads of A land in registers that the MFMAs read directly, and a third (check_lds_order, `--lds-order file.s`)
+the GEMM of bfp_matmul_bf16.hip, whose inline LDS reads are waited for a slab at a time; they are described at the functions.
 """
 from __future__ import annotations
 
@@ -96,8 +97,7 @@ def _blocks(body):
     return blocks
 
 
-def _check_kernel(name, body, problems, release_on_mfma=False):
-    blocks = _blocks(body)
+def _successors(name, blocks, problems):
     index = {b["label"]: i for i, b in enumerate(blocks) if b["label"] is not None}
     succs = []
     for i, b in enumerate(blocks):
@@ -112,6 +112,12 @@ def _check_kernel(name, body, problems, release_on_mfma=False):
                 else:
                     out.append(index[t])
         succs.append(out)
+    return succs
+
+
+def _check_kernel(name, body, problems, release_on_mfma=False):
+    blocks = _blocks(body)
+    succs = _successors(name, blocks, problems)
     n_ring = sum(1 for b in blocks for t, a in b["instrs"] if a and t.startswith("global_load_dwordx4") and "sc1" not in t)
     if not n_ring:
         problems.append(f"{name}: no hand-written activation loads found (has the kernel changed?)")
@@ -152,7 +158,11 @@ def _check_kernel(name, body, problems, release_on_mfma=False):
                 report.append(f"{name}: registers {sorted(ring | slot | lds)} still have a load in flight at s_endpgm")
         return frozenset(ring), frozenset(slot), frozenset(lds)
 
-    empty = (frozenset(), frozenset(), frozenset())
+    _propagate(blocks, succs, (frozenset(), frozenset(), frozenset()), run, lambda p, q: tuple(a | b for a, b in zip(p, q)), problems)
+
+
+def _propagate(blocks, succs, empty, run, merge, problems):
+    """Carries the state through the control-flow graph until nothing changes, then reports what every block finds."""
     state_in = [None] * len(blocks)
     state_in[0] = empty
     work = [0]
@@ -160,7 +170,7 @@ def _check_kernel(name, body, problems, release_on_mfma=False):
         i = work.pop()
         out = run(blocks[i], state_in[i], None)
         for j in succs[i]:
-            merged = out if state_in[j] is None else tuple(a | b for a, b in zip(state_in[j], out))
+            merged = out if state_in[j] is None else merge(state_in[j], out)
             if merged != state_in[j]:
                 state_in[j] = merged
                 work.append(j)
@@ -212,5 +222,62 @@ def check_ring_operands(path: str, kernel_substrings=("matmul_tall_kernel",)) ->
     return len(problems)
 
 
+_QUEUE = 64      # LDS operations told apart; older ones share the last place
+
+
+def _check_lds_order(name, body, problems):
+    blocks = _blocks(body)
+    succs = _successors(name, blocks, problems)
+    if not any(a and t.startswith("ds_read") for b in blocks for t, a in b["instrs"]):
+        problems.append(f"{name}: no hand-written LDS reads found (has the kernel changed?)")
+
+    def run(block, state, report):
+        queue = list(state)                                                  # registers of every LDS operation in flight, youngest first
+        for text, asm in block["instrs"]:
+            wait = re.search(r"lgkmcnt\((\d+)\)", text) if text.startswith("s_waitcnt") else None
+            if wait:
+                del queue[int(wait.group(1)):]
+                continue
+            flying = frozenset().union(*queue)
+            # an operation that reads its own address out of the register it loads is fine: the address goes with it
+            hit = _regs(text) & flying
+            if hit and report is not None:
+                report.append(f"{name}: instruction touches registers {sorted(hit)} while a hand-scheduled LDS read into them is in flight: {text}")
+            if text.startswith("ds_"):
+                queue.insert(0, _regs(text.split(",")[0]) if asm and text.startswith("ds_read") else frozenset())
+                if len(queue) > _QUEUE:
+                    queue[_QUEUE - 1:] = [queue[_QUEUE - 1] | queue[_QUEUE]]
+            if text.startswith("s_endpgm") and flying and report is not None:
+                report.append(f"{name}: registers {sorted(flying)} still have an LDS read in flight at s_endpgm")
+        return tuple(queue)
+
+    def merge(p, q):
+        short, long = sorted((p, q), key=len)
+        return tuple(a | b for a, b in zip(short, long)) + long[len(short):]
+
+    _propagate(blocks, succs, (), run, merge, problems)
+
+
+def check_lds_order(path: str, kernel_substrings=("matmul_direct_kernel",)) -> int:
+    """The GEMM of bfp_matmul_bf16.hip reads all operands of a step out of LDS with inline `ds_read*` and waits for them itself,
+    first with `s_waitcnt lgkmcnt(N)`, N the reads of the second slab.  LDS operations return in order, so behind lgkmcnt(N) all
+    but the youngest N have landed, whoever issued them (scalar loads count too and return in any order, which leaves fewer
+    of the N to LDS operations, never more).  Any instruction that names a register in flight (a copy, a spill, a reuse, a use in
+    front of the wait) fails the build, and so does a read still in flight when the kernel ends."""
+    problems, checked = [], 0
+    with open(path) as f:
+        lines = f.read().split("\n")
+    for name, body in _kernels(lines):
+        if any(k in name for k in kernel_substrings):
+            checked += 1
+            _check_lds_order(name, body, problems)
+    if not checked:
+        problems.append(f"no kernel matching {kernel_substrings} in {path}")
+    for p in problems[:40]:
+        print("check_isa:", p, file=sys.stderr)
+    return len(problems)
+
+
 if __name__ == "__main__":
-    sys.exit(1 if (check_ring_operands(sys.argv[2]) if sys.argv[1] == "--ring-operands" else check(sys.argv[1])) else 0)
+    _FORMS = {"--ring-operands": check_ring_operands, "--lds-order": check_lds_order}
+    sys.exit(1 if (_FORMS[sys.argv[1]](sys.argv[2]) if sys.argv[1] in _FORMS else check(sys.argv[1])) else 0)
