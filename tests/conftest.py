@@ -22,7 +22,7 @@ def oracle():
 
 
 # knobs of libttmi's test entry point (tt-metal_amd/csrc/ttmi_internal.h: TTMI_KNOB_*)
-KNOB = {"kernel": 0, "workgroups": 1, "block": 2, "spin_limit": 3, "drop_partial_sums": 4, "xcds": 5}
+KNOB = {"kernel": 0, "workgroups": 1, "block": 2, "spin_limit": 3, "drop_partial_sums": 4, "xcds": 5, "scratch_limit": 6}
 KERNEL_CODE = {"stream": 1, "wide": 2, "tile": 3, "expanded": 4, "bf16 in place": 5}
 
 
@@ -44,7 +44,7 @@ def test_library():
 @pytest.fixture
 def knobs(test_library):
     """knobs(name, value) on the library's test entry point (name: kernel = stream | wide | tile | expanded | bf16 in place, workgroups,
-    block = 256 | 128 | 64 | 4 | 384, spin_limit, drop_partial_sums, xcds = 1 | 8); everything set is cleared again after the test."""
+    block = 256 | 128 | 64 | 4 | 384, spin_limit, drop_partial_sums, xcds = 1 | 8, scratch_limit in bytes); everything set is cleared again after the test."""
     import ctypes
 
     from ttmi import capi

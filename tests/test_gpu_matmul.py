@@ -284,6 +284,83 @@ def test_decode_gemm_in_a_hip_graph(oracle):
         assert torch.equal(other.view(torch.int16), eager.view(torch.int16))
 
 
+@pytest.mark.parametrize("batch,b_batch,m,k,n", [(8, 1, 384, 1024, 4096), (12, 12, 384, 1024, 1024), (5, 1, 333, 512, 2112)])
+def test_kernels_without_scratch_in_hip_graphs(batch, b_batch, m, k, n, test_library):
+    """Shapes of the tiled kernels captured with no workspace on a stream that has no scratch: nothing is allocated, two graphs
+    captured on that one stream run side by side on two others, and both still do when the library's scratch has been released
+    and eager calls (which may take a kernel with scratch) run in between.  The captured sums need not be in the eager order:
+    2 k 2^-24 of the terms on either side."""
+    L = test_library
+    L.ttmi_test_allocations.restype = ctypes.c_uint64
+    assert L.ttmi_test_kernel_choice(batch, m, k, n, BFP8, capi.FLOAT32) == 3
+    words, outs, graphs, want, terms = [], [], [], [], []
+    a = bf16_dev(workloads.activations_bf16(m, k, seed=600, batch=batch)).reshape(batch, m, k)
+    for i in range(2):
+        words.append(capi.pack_tensor(BFP8, torch.from_numpy(workloads.weights_f32(k, n, seed=601 + i, batch=b_batch)).cuda().reshape(b_batch, k, n)))
+        w = capi.unpack_tensor(BFP8, words[i], (b_batch, k, n)).expand(batch, k, n)
+        want.append(torch.stack([a[s].double() @ w[s].double() for s in range(batch)]))
+        terms.append(torch.stack([a[s].double().abs() @ w[s].double().abs() for s in range(batch)]))
+        outs.append(torch.zeros(batch, m, n, device="cuda"))
+    capi.device_status()
+    torch.cuda.synchronize()
+    capi.release_scratch()
+    side, made = torch.cuda.Stream(), L.ttmi_test_allocations()
+    for i in range(2):
+        graphs.append(torch.cuda.CUDAGraph())
+        with torch.cuda.graph(graphs[i], stream=side):
+            capi.check(L.ttmi_matmul_bfp(a.data_ptr(), capi.ROW_MAJOR, words[i].data_ptr(), BFP8, batch, b_batch, m, k, n, None, capi.ACT_NONE,
+                                         outs[i].data_ptr(), capi.ROW_MAJOR, capi.FLOAT32, None, 0, side.cuda_stream))
+    assert L.ttmi_test_allocations() == made
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    for replay in range(4):
+        for out in outs:
+            out.zero_()
+        torch.cuda.synchronize()
+        for graph, stream in zip(graphs, streams):
+            with torch.cuda.stream(stream):
+                graph.replay()
+        torch.cuda.synchronize()
+        eager = capi.matmul_bfp(a, capi.ROW_MAJOR, words[replay % 2], BFP8, batch, b_batch, m, k, n, out_dtype=torch.float32)
+        for i, c in [(0, outs[0]), (1, outs[1]), (replay % 2, eager.reshape(batch, m, n))]:
+            assert bool(((c.double() - want[i]).abs() <= 2.0 * k * 2.0 ** -24 * terms[i]).all()), (replay, i)
+        if replay == 1:
+            torch.cuda.synchronize()
+            capi.release_scratch()
+
+
+@pytest.mark.parametrize("batch,b_batch,m,k,n", [(8, 1, 384, 1024, 4096), (12, 12, 384, 1024, 1024)])
+def test_without_memory_for_scratch_the_kernel_that_needs_none_runs(batch, b_batch, m, k, n, knobs):
+    """A device that refuses the library any buffer: shapes that a kernel without scratch can do are done by that one, with the
+    bits of the call that may not allocate, and the refusal is not reported by a later call."""
+    a = bf16_dev(workloads.activations_bf16(m, k, seed=610, batch=batch)).reshape(batch, m, k)
+    words = capi.pack_tensor(BFP8, torch.from_numpy(workloads.weights_f32(k, n, seed=611, batch=b_batch)).cuda().reshape(b_batch, k, n))
+    want = torch.empty(batch, m, n, device="cuda")
+    capi.check(capi.lib().ttmi_matmul_bfp_static(a.data_ptr(), capi.ROW_MAJOR, words.data_ptr(), BFP8, batch, b_batch, m, k, n, None, capi.ACT_NONE, want.data_ptr(),
+                                                 capi.ROW_MAJOR, capi.FLOAT32, torch.cuda.current_stream().cuda_stream))
+    torch.cuda.synchronize()
+    capi.release_scratch()
+    knobs("scratch_limit", 0)
+    for _ in range(2):
+        got = capi.matmul_bfp(a, capi.ROW_MAJOR, words, BFP8, batch, b_batch, m, k, n, out_dtype=torch.float32)
+        assert torch.equal(got.reshape(batch, m, n), want)
+
+
+def test_without_memory_for_partial_sums_nothing_is_cut(knobs):
+    """Memory for the expanded weights alone: the bits of a caller's workspace of that size, in one piece per output."""
+    batch, m, k, n = 1, 260, 2080, 256
+    a = bf16_dev(workloads.activations_bf16(m, k, seed=620)).reshape(batch, m, k)
+    words = capi.pack_tensor(BFP8, torch.from_numpy(workloads.weights_f32(k, n, seed=621)).cuda().reshape(1, k, n))
+    knobs("kernel", "expanded")
+    need = capi.lib().ttmi_matmul_bfp_workspace_bytes(batch, m, k, n, BFP8)
+    call = lambda **more: capi.matmul_bfp(a, capi.ROW_MAJOR, words, BFP8, 1, 1, m, k, n, out_dtype=torch.float32, **more)
+    want = call(workspace=torch.empty(need, dtype=torch.uint8, device="cuda"))
+    cut = call()
+    torch.cuda.synchronize()
+    capi.release_scratch()
+    knobs("scratch_limit", need)
+    assert torch.equal(call(), want) and not torch.equal(cut, want)
+
+
 @pytest.mark.parametrize("kernel", ["stream", "wide"])
 @pytest.mark.parametrize("fmt", [BFP8, BFP4])
 def test_row_exponents_over_the_whole_range(oracle, kernel, fmt, knobs):

@@ -1222,6 +1222,22 @@ static bool fold_batch(const MatmulArgs &x, bool c_bfp) {
     return folded.us < choose_kernel_own_scratch(x.batch, 1, x.m, x.k, x.n, x.b_fmt, c_bfp).us;
 }
 
+// Whether a call may go to `best` (as `batch` slices of `m` rows), which keeps expanded weights in scratch of the library's own,
+// instead of to `plain`, where it goes with any scratch.  Not without memory for them.  In a capture nothing can
+// be allocated, and what is recorded may be replayed on any stream beside any other: a kernel without scratch stays so, and
+// one with is exchanged for the route that the same call takes outside a capture only where that has left its buffer.
+static bool scratch_for(Kernel best, uint32_t batch, uint32_t m, Kernel plain, const MatmulArgs &x, hipStream_t st) {
+    if (best != Kernel::Expanded && best != Kernel::Direct) return true;
+    const size_t need = best == Kernel::Expanded ? matmul_expanded_scratch_bytes(batch, x.b_batch, m, x.k, x.n) : matmul_direct_scratch_bytes(x.b_batch, x.k, x.n);
+    if (stream_is_capturing(st)) {
+        const bool shares_outputs = (plain == Kernel::Wide || plain == Kernel::Stream) && decompose(x.batch, x.m, x.k, x.n, plain == Kernel::Wide).split > 1;
+        return (shares_outputs || plain == Kernel::Expanded) && scratch_held(SCRATCH_EXPANDED, st, need);
+    }
+    void *ignored;
+    bool fresh;
+    return scratch_held(SCRATCH_EXPANDED, st, need) || scratch_get(SCRATCH_EXPANDED, st, need, &ignored, &fresh) == TTMI_OK;
+}
+
 size_t matmul_gated_workspace_bytes(uint32_t batch, uint32_t m, uint32_t k, uint32_t n) {
     if (!batch || !m || !k || !n) return 0;
     return slot_bytes_needed(decompose(batch, m, k, n, true, true), true, true);
@@ -1270,11 +1286,14 @@ int matmul_bfp(const MatmulArgs &asked, hipStream_t st) {
     // every kernel but the 64-column one packs a block-float output in its epilogue (choose_kernel keeps that one out of it)
     const bool c_bfp = x.c_dtype == TTMI_BFLOAT8_B || x.c_dtype == TTMI_BFLOAT4_B;
     const bool a8 = x.a_dtype == TTMI_BFLOAT8_B;      // block-float activations: the 128-column kernel alone takes them
+    Kernel kernel = choose_kernel(x.batch, x.m, x.k, x.n, x.b_fmt, c_bfp || a8);
     // (the workspace query answers for the slices as they are, so a caller's workspace serves those)
-    const bool own_scratch = !x.workspace && !x.no_alloc;
-    if (own_scratch && !a8 && fold_batch(x, c_bfp)) { x.m *= x.batch; x.batch = 1; }
-    const Kernel kernel = own_scratch ? choose_kernel_own_scratch(x.batch, x.b_batch, x.m, x.k, x.n, x.b_fmt, c_bfp || a8).kernel
-                                      : choose_kernel(x.batch, x.m, x.k, x.n, x.b_fmt, c_bfp || a8);
+    if (!x.workspace && !x.no_alloc && !a8) {
+        const bool folded = fold_batch(x, c_bfp);
+        const uint32_t batch = folded ? 1 : x.batch, m = folded ? x.batch * x.m : x.m;
+        const Kernel best = choose_kernel_own_scratch(batch, x.b_batch, m, x.k, x.n, x.b_fmt, c_bfp).kernel;
+        if ((folded || best != kernel) && scratch_for(best, batch, m, kernel, x, st)) { kernel = best; x.batch = batch; x.m = m; }
+    }
     if (a8 && !matmul_takes_bfp_activations(x.batch, x.m, x.k, x.n, x.b_fmt))
         return fail(TTMI_ERR_UNSUPPORTED, "matmul: block-float activations are taken by the one-band streaming kernel only, which this shape does "
                     "not go to (ttmi_matmul_bfp_ab_supported): expand them with ttmi_typecast_tiles first");

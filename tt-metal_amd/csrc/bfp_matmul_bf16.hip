@@ -329,6 +329,8 @@ double matmul_direct_estimate(uint32_t batch, uint32_t b_batch, uint32_t m, uint
     return 5.0 + (double)b_batch * k * n * (bytes_per_weight + 2.0) / 4.0e6 + direct_us(batch, m, k, n, nullptr);
 }
 
+size_t matmul_direct_scratch_bytes(uint32_t b_batch, uint32_t k, uint32_t n) { return (size_t)b_batch * (k / 32) * (n / 32) * 2048; }
+
 int matmul_bf16_direct(const MatmulArgs &x, hipStream_t st) {
     DirectDev p{};
     p.a = (const uint8_t *)x.a; p.b = (const uint8_t *)x.b; p.bias = (const uint16_t *)x.bias; p.c = (uint8_t *)x.c;
@@ -342,7 +344,7 @@ int matmul_bf16_direct(const MatmulArgs &x, hipStream_t st) {
         if (blocks > 0x7fffffffull) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: problem too large for one launch");
         void *dense;
         bool fresh;
-        if (int rc = scratch_get(SCRATCH_EXPANDED, st, (size_t)pieces * 16, &dense, &fresh)) return rc;
+        if (int rc = scratch_get(SCRATCH_EXPANDED, st, matmul_direct_scratch_bytes(x.b_batch, x.k, x.n), &dense, &fresh)) return rc;
         if (x.b_fmt == TTMI_BFLOAT8_B)
             hipLaunchKernelGGL((expand_tiles_kernel<7>), dim3((uint32_t)blocks), dim3(256), 0, st, p.b, (u32x4 *)dense, pieces);
         else

@@ -385,6 +385,11 @@ size_t matmul_expanded_workspace_bytes(uint32_t b_batch, uint32_t k, uint32_t n)
     return (size_t)((uint64_t)b_batch * (k / 32) * groups * GROUP_BYTES);
 }
 
+static size_t aligned_weights_bytes(uint32_t b_batch, uint32_t k, uint32_t n) { return (matmul_expanded_workspace_bytes(b_batch, k, n) + 255) & ~(size_t)255; }
+size_t matmul_expanded_scratch_bytes(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n) {
+    return aligned_weights_bytes(b_batch, k, n) + plan_expanded(batch, b_batch, m, k, n, 0, true).parts_bytes;
+}
+
 // What the launches below, and the kernel that reads bf16 weights in place, cannot take.
 int validate_expanded(const MatmulArgs &x) {
     const uint64_t kt = x.k / 32, groups = ((uint64_t)x.n / 32 + 1) / 2;
@@ -415,13 +420,20 @@ int matmul_bfp_expanded(const MatmulArgs &x, hipStream_t st) {
     p.c_bfp = x.c_dtype == TTMI_BFLOAT8_B ? 7 : x.c_dtype == TTMI_BFLOAT4_B ? 3 : 0;
     const uint64_t items = (uint64_t)x.b_batch * p.kt * p.groups;
     if (int rc = validate_expanded(x)) return rc;
-    const size_t weights_bytes = (matmul_expanded_workspace_bytes(x.b_batch, x.k, x.n) + 255) & ~(size_t)255;
+    const size_t weights_bytes = aligned_weights_bytes(x.b_batch, x.k, x.n);
     ExpandedPlan e = plan_expanded(x.batch, x.b_batch, x.m, x.k, x.n, 0, true);
     void *expanded = x.workspace;
     if (!expanded) {
-        // the library's own buffer, one per stream (launches on one stream run in order, so they can share it)
+        // the library's own buffer, one per stream (launches on one stream run in order, so they can share it).  Room for the
+        // weights is what a call needs: where there is no more to be had (no memory, or a capture that the buffer at hand is to
+        // serve) nothing is cut.
         bool fresh;
-        if (int rc = scratch_get(SCRATCH_EXPANDED, st, weights_bytes + e.parts_bytes, &expanded, &fresh)) return rc;
+        const bool only_weights = e.parts_bytes && !scratch_held(SCRATCH_EXPANDED, st, weights_bytes + e.parts_bytes) &&
+                                  scratch_held(SCRATCH_EXPANDED, st, weights_bytes) && stream_is_capturing(st);
+        if (only_weights || scratch_get(SCRATCH_EXPANDED, st, weights_bytes + e.parts_bytes, &expanded, &fresh)) {
+            e = plan_expanded(x.batch, x.b_batch, x.m, x.k, x.n, 0, false);
+            if (int rc = scratch_get(SCRATCH_EXPANDED, st, weights_bytes, &expanded, &fresh)) return rc;
+        }
     } else if (x.workspace_bytes < weights_bytes + e.parts_bytes) {
         e = plan_expanded(x.batch, x.b_batch, x.m, x.k, x.n, 0, false);      // a caller's workspace has to hold the weights; partial sums only if they fit
     }

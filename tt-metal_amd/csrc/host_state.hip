@@ -51,7 +51,12 @@ int scratch_get(int kind, hipStream_t stream, size_t bytes, void **ptr, bool *fr
     if (b.bytes < bytes) {
         const size_t size = scratch_grown_size(b.bytes, bytes);
         void *p = nullptr;
-        if (int rc = check_hip(hipMalloc(&p, size), "hipMalloc(library scratch)")) return rc;
+        uint32_t limit;
+        const bool refused = knob(TTMI_KNOB_SCRATCH_LIMIT, &limit) && size > limit;
+        if (int rc = check_hip(refused ? hipErrorOutOfMemory : hipMalloc(&p, size), "hipMalloc(library scratch)")) {
+            (void)hipGetLastError();                 // reported here, not by the next launch
+            return rc;
+        }
         ++g_allocations;
         if (b.ptr) g_retired.push_back(Retired{b.ptr, b.bytes, dev});
         b.ptr = p; b.bytes = size;
@@ -61,6 +66,23 @@ int scratch_get(int kind, hipStream_t stream, size_t bytes, void **ptr, bool *fr
     *ptr = b.ptr;
     if (capacity) *capacity = b.bytes;
     return TTMI_OK;
+}
+
+bool scratch_held(int kind, hipStream_t stream, size_t bytes) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return false;
+    std::lock_guard<std::mutex> lock(g_guard);
+    const auto it = g_live.find(Key{kind, dev, stream});
+    return it != g_live.end() && it->second.bytes >= bytes;
+}
+
+bool stream_is_capturing(hipStream_t stream) {
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &status) != hipSuccess) {       // the default stream while another one is captured
+        (void)hipGetLastError();
+        return true;
+    }
+    return status != hipStreamCaptureStatusNone;
 }
 
 uint64_t scratch_generation(int kind) {

@@ -20,6 +20,8 @@ enum { SCRATCH_SLOTS = 0, SCRATCH_EXPANDED = 1, SCRATCH_KINDS = 2 };
 // set when the contents are undefined (a new buffer, or one invalidated since): the caller initialises ALL of it on `stream`
 // (*capacity bytes: buffers grow geometrically, so a later, larger request may be served without being fresh).
 int scratch_get(int kind, hipStream_t stream, size_t bytes, void **ptr, bool *fresh, size_t *capacity = nullptr);
+bool scratch_held(int kind, hipStream_t stream, size_t bytes);      // scratch_get would allocate nothing
+bool stream_is_capturing(hipStream_t stream);
 void scratch_invalidate(int kind);
 uint64_t scratch_generation(int kind);      // raised by scratch_invalidate
 size_t scratch_grown_size(size_t have, size_t need);
@@ -35,7 +37,8 @@ enum {
     TTMI_KNOB_SPIN_LIMIT = 3,         // polls before a bounded wait gives up
     TTMI_KNOB_DROP_PARTIAL_SUMS = 4,  // producers do not publish their partial sums (so that a wait must give up)
     TTMI_KNOB_XCDS = 5,               // 1: the 128-column kernel assumes nothing about where workgroups run (device-scope hand-over)
-    TTMI_KNOB_COUNT = 6
+    TTMI_KNOB_SCRATCH_LIMIT = 6,      // a library buffer of more bytes than that is refused as by a device without memory
+    TTMI_KNOB_COUNT = 7
 };
 #ifdef TTMI_TEST_HOOKS
 bool knob(int which, uint32_t *value);
@@ -99,5 +102,7 @@ double matmul_direct_estimate(uint32_t batch, uint32_t b_batch, uint32_t m, uint
 int validate_expanded(const MatmulArgs &args);
 double matmul_expanded_estimate(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, double bytes_per_weight);   // us, k ranges cut where that helps
 size_t matmul_expanded_workspace_bytes(uint32_t b_batch, uint32_t k, uint32_t n);
+size_t matmul_expanded_scratch_bytes(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n);      // with the partial sums of k ranges
+size_t matmul_direct_scratch_bytes(uint32_t b_batch, uint32_t k, uint32_t n);       // bf16 tiles of block-float weights
 
 }  // namespace ttmi
