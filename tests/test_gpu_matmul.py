@@ -345,6 +345,39 @@ def test_without_memory_for_scratch_the_kernel_that_needs_none_runs(batch, b_bat
         assert torch.equal(got.reshape(batch, m, n), want)
 
 
+@pytest.mark.parametrize("kernel", ["expanded", "bf16 in place"])
+def test_host_threads_on_one_stream(kernel, knobs):
+    """Three host threads that launch on one stream, each with weights of its own, while the library's buffer holds one call's
+    expanded weights at a time: every output has the bits of the same call alone."""
+    import threading
+
+    knobs("kernel", kernel)
+    m, k, n, calls = 260, 1056, 512, 40
+    a = bf16_dev(workloads.activations_bf16(m, k, seed=630))
+    words = [capi.pack_tensor(BFP8, torch.from_numpy(workloads.weights_f32(k, n, seed=631 + i)).cuda().reshape(1, k, n)) for i in range(3)]
+    want = [capi.matmul_bfp(a, capi.ROW_MAJOR, w, BFP8, 1, 1, m, k, n, out_dtype=torch.float32) for w in words]
+    outs = [torch.empty(calls, m, n, device="cuda") for _ in words]
+    stream, failed, together = torch.cuda.current_stream().cuda_stream, [], threading.Barrier(3)
+    torch.cuda.synchronize()
+
+    def launch(i):
+        together.wait()
+        for c in range(calls):
+            if capi.lib().ttmi_matmul_bfp(a.data_ptr(), capi.ROW_MAJOR, words[i].data_ptr(), BFP8, 1, 1, m, k, n, None, capi.ACT_NONE, outs[i][c].data_ptr(),
+                                          capi.ROW_MAJOR, capi.FLOAT32, None, 0, stream):
+                failed.append(i)
+
+    threads = [threading.Thread(target=launch, args=(i,)) for i in range(3)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    torch.cuda.synchronize()
+    assert not failed
+    for i in range(3):
+        assert bool((outs[i] == want[i].reshape(1, m, n)).all()), i
+
+
 def test_without_memory_for_partial_sums_nothing_is_cut(knobs):
     """Memory for the expanded weights alone: the bits of a caller's workspace of that size, in one piece per output."""
     batch, m, k, n = 1, 260, 2080, 256

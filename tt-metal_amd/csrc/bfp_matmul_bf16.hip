@@ -339,11 +339,13 @@ int matmul_bf16_direct(const MatmulArgs &x, hipStream_t st) {
     p.a_tiled = x.a_layout == TTMI_TILE; p.c_tiled = x.c_layout == TTMI_TILE; p.c_f32 = x.c_dtype == TTMI_FLOAT32;
     p.c_bfp = x.c_dtype == TTMI_BFLOAT8_B ? 7 : x.c_dtype == TTMI_BFLOAT4_B ? 3 : 0;
     p.unscale = 1.0f;
+    std::unique_lock<std::mutex> launches(expanded_scratch_guard(), std::defer_lock);
     if (x.b_fmt != TTMI_BFLOAT16) {                             // scratch of the library's own, which callers without it do not come here for
         const uint64_t pieces = (uint64_t)x.b_batch * p.kt * p.nt * 128, blocks = (pieces + 1023) / 1024;
         if (blocks > 0x7fffffffull) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: problem too large for one launch");
         void *dense;
         bool fresh;
+        launches.lock();
         if (int rc = scratch_get(SCRATCH_EXPANDED, st, matmul_direct_scratch_bytes(x.b_batch, x.k, x.n), &dense, &fresh)) return rc;
         if (x.b_fmt == TTMI_BFLOAT8_B)
             hipLaunchKernelGGL((expand_tiles_kernel<7>), dim3((uint32_t)blocks), dim3(256), 0, st, p.b, (u32x4 *)dense, pieces);

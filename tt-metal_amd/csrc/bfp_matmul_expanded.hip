@@ -423,7 +423,9 @@ int matmul_bfp_expanded(const MatmulArgs &x, hipStream_t st) {
     const size_t weights_bytes = aligned_weights_bytes(x.b_batch, x.k, x.n);
     ExpandedPlan e = plan_expanded(x.batch, x.b_batch, x.m, x.k, x.n, 0, true);
     void *expanded = x.workspace;
+    std::unique_lock<std::mutex> launches(expanded_scratch_guard(), std::defer_lock);
     if (!expanded) {
+        launches.lock();
         // the library's own buffer, one per stream (launches on one stream run in order, so they can share it).  Room for the
         // weights is what a call needs: where there is no more to be had (no memory, or a capture that the buffer at hand is to
         // serve) nothing is cut.

@@ -76,6 +76,11 @@ bool scratch_held(int kind, hipStream_t stream, size_t bytes) {
     return it != g_live.end() && it->second.bytes >= bytes;
 }
 
+std::mutex &expanded_scratch_guard() {
+    static std::mutex guard;
+    return guard;
+}
+
 bool stream_is_capturing(hipStream_t stream) {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(stream, &status) != hipSuccess) {       // the default stream while another one is captured

@@ -4,6 +4,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <mutex>
+
 #include "ttmi.h"
 
 namespace ttmi {
@@ -22,6 +24,9 @@ enum { SCRATCH_SLOTS = 0, SCRATCH_EXPANDED = 1, SCRATCH_KINDS = 2 };
 int scratch_get(int kind, hipStream_t stream, size_t bytes, void **ptr, bool *fresh, size_t *capacity = nullptr);
 bool scratch_held(int kind, hipStream_t stream, size_t bytes);      // scratch_get would allocate nothing
 bool stream_is_capturing(hipStream_t stream);
+// Held from scratch_get(SCRATCH_EXPANDED) to the last launch that reads the buffer: one launch of a call fills it, the next ones
+// read it, and what another host thread launches on the same stream must not come between.
+std::mutex &expanded_scratch_guard();
 void scratch_invalidate(int kind);
 uint64_t scratch_generation(int kind);      // raised by scratch_invalidate
 size_t scratch_grown_size(size_t have, size_t need);
