@@ -968,6 +968,26 @@ def test_slices_that_share_their_weights(batch, m, k, n):
         assert torch.equal(capi.untilize(tiles, (batch, m, n)).view(torch.int16), c.bfloat16().view(torch.int16))
 
 
+@pytest.mark.parametrize("kernel", ["expanded", "bf16 in place"])
+def test_bf16_weights_whose_tile_rows_exceed_4_gib(kernel, knobs):
+    """2^26 + 32 columns: a tile row of the weights is 4 GiB and one tile, so the offset of the next one, and of the last column,
+    takes more than 32 bits.  Float64 with the fp32 accumulation bound at the first, the last and some middle tiles of columns."""
+    m, k, n = 32, 96, (1 << 26) + 32
+    if torch.cuda.mem_get_info()[0] < 64 << 30:
+        pytest.skip("needs 34 GiB of device memory")
+    tiles = torch.randn((k // 32, n // 32, 2, 2, 16, 16), device="cuda", dtype=torch.bfloat16, generator=torch.Generator(device="cuda").manual_seed(540))
+    a = bf16_dev(workloads.activations_bf16(m, k, seed=541)).reshape(1, m, k)
+    knobs("kernel", kernel)
+    c = capi.matmul_bf16(a, capi.ROW_MAJOR, tiles.view(torch.int16).view(torch.uint8), 1, 1, m, k, n, out_dtype=torch.float32)[0]
+    for t in (0, 1, 12345, (1 << 20) - 1, 1 << 20, (1 << 21) - 1, 1 << 21):
+        w = tiles[:, t].permute(0, 1, 3, 2, 4).reshape(k, 32)
+        check_on_device(c[:, t * 32 : t * 32 + 32], a[0], w, k)
+    torch.cuda.synchronize()
+    del tiles, c
+    capi.release_scratch()
+    torch.cuda.empty_cache()
+
+
 @pytest.mark.parametrize("block", [64, 128])
 @pytest.mark.parametrize("batch,b_batch,m,k,n", [(1, 1, 1, 32, 32), (1, 1, 33, 64, 96), (2, 2, 127, 96, 160), (3, 1, 160, 128, 288), (17, 17, 64, 160, 64)])
 def test_bf16_weights_read_in_place(oracle, batch, b_batch, m, k, n, block, knobs):

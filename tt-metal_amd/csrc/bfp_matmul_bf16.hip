@@ -88,7 +88,7 @@ __global__ __launch_bounds__(256, 2) void matmul_direct_kernel(const DirectDev p
 
     // ---- requests: piece i of this wavefront is half a tile, 16 bytes per lane --------------------------------------------
     const uint8_t *src[LOADS];
-    uint32_t step[LOADS];
+    uint64_t step[LOADS];                                       // a k tile row of B has more than 4 GiB from 2^26 columns on
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) {
         const uint32_t piece = wave * LOADS + i, tile = piece >> 1, at = (piece & 1) * 64 + lane;   // 16-byte place in the tile
@@ -107,7 +107,7 @@ __global__ __launch_bounds__(256, 2) void matmul_direct_kernel(const DirectDev p
         } else {
             const uint32_t col = min(nt0 + tile - BANDS, p.nt - 1);
             src[i] = p.b + ((uint64_t)(p.b_batch == 1 ? 0 : bb) * p.kt * p.nt + col) * 2048 + face * 512 + (within ^ ((face & 1) * 8)) * 16;
-            step[i] = p.nt * 2048;
+            step[i] = (uint64_t)p.nt * 2048;
         }
     }
     auto request = [&](uint32_t stage) __attribute__((always_inline)) {

@@ -208,15 +208,14 @@ __global__ __launch_bounds__(512, 1) void matmul_expanded_kernel(const ExpandedD
         const uint32_t kq = (lane & 3) ^ ((lane >> 4) & 3);              // XOR swizzle of the row's four 16-byte chunks
         if (p.a_tiled) a_off[i] = (row >> 5) * p.kt * 2048 + (((row >> 4) & 1) * 2 + (kq >> 1)) * 512 + (row & 15) * 32 + (kq & 1) * 16;
         else a_off[i] = (row * p.k + kq * 8) * 2;
-        const uint32_t kb = wave * 2 + i;                                 // group kb / 4 of the block, KB kb % 4 of it
-        const uint32_t group = min(tn * 4 + kb / 4, p.groups - 1);        // past the last group: any valid memory
-        b_off[i] = group * GROUP_BYTES + (kb & 3) * 1024 + lane * 16;
+        b_off[i] = ((wave & 1) * 2 + i) * 1024 + lane * 16;               // KB of the wavefront's group
     }
     const uint8_t *a_base;
     uint32_t a_step;
     if (p.a_tiled) { a_base = p.a + (uint64_t)bb * ((p.m + 31) / 32) * p.kt * 2048; a_step = 2048; }
     else { a_base = p.a + (uint64_t)bb * p.m * p.k * 2; a_step = 64; }
-    const uint8_t *w_base = p.w + (uint64_t)(p.b_batch == 1 ? 0 : bb) * p.kt * p.groups * GROUP_BYTES;
+    const uint32_t group = min(tn * 4 + wave / 2, p.groups - 1);          // past the last group: any valid memory
+    const uint8_t *w_base = p.w + ((uint64_t)(p.b_batch == 1 ? 0 : bb) * p.kt * p.groups + group) * GROUP_BYTES;      // 4 GiB and more from 2^26 columns on
     const uint64_t w_step = (uint64_t)p.groups * GROUP_BYTES;
     // request j of a step: j = 0, 1 the wavefront's A rows, j = 2, 3 its B KBs (steps past the end re-request the last one)
     auto request_one = [&](uint32_t kstep, int j) __attribute__((always_inline)) {
