@@ -347,3 +347,14 @@ def test_large_tensors_from_and_to_host_memory(device, shape, name, source):
     assert torch.equal(ttnn.to_torch(on_host), back)
     pinned = ttnn.from_torch(host.pin_memory(), dtype=dtype, layout=ttnn.TILE_LAYOUT, device=device)
     assert torch.equal(pinned._buf.view(torch.int32).cpu(), want.cpu())
+
+
+def test_pinned_slots_are_coherent(device, test_library):
+    """Host and kernels exchange the slots of a large transfer while other kernels run, so the slots' allocation states coherence
+    itself (flag 0x40000000, hipHostMallocCoherent): what the runtime takes when neither flag is given is the environment's."""
+    import ttnn
+    from ttmi import pybind
+
+    t = ttnn.from_torch(torch.randn(1, 1, 2048, 1024), dtype=ttnn.bfloat8_b, layout=ttnn.TILE_LAYOUT, device=device)
+    ttnn.to_torch(t)
+    assert pybind.module("_ttmi_test").test_slot_flags() & 0x40000000

@@ -5,7 +5,7 @@
 
 Next to them a test build of both: libttmi_test.so is the same sources with -DTTMI_TEST_HOOKS, which adds the entry points
 ttmi_test_* (forcing a kernel, a decomposition, a give-up; reading the host's index functions) that the product library
-does not have, and _ttmi_test is the same bindings over it.  Only tests load those two.
+does not have, and _ttmi_test is the same bindings over it (with one entry of its own, what the pinned slots were allocated with).  Only tests load those two.
 """
 from __future__ import annotations
 
@@ -109,7 +109,7 @@ def build_bindings(force: bool = False, verbose: bool = False) -> str:
         first = first or out
         if force or _stale(out, deps):
             cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-shared", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__",
-                   "-DTTMI_PYBIND_NAME=" + name,
+                   "-DTTMI_PYBIND_NAME=" + name] + (["-DTTMI_TEST_HOOKS"] if lib_path == LIB_TEST else []) + [
                    "-I", pybind11.get_include(), "-I", sysconfig.get_paths()["include"], "-I", os.path.join(ROOT, "include"), "-I", CSRC,
                    "-I", os.path.join(rocm, "include")] + sources + [
                    "-o", out, "-L", LIB_DIR, "-l" + lib_name, "-L", os.path.join(rocm, "lib"), "-lamdhip64", "-Wl,-rpath,$ORIGIN", "-Wl,-rpath," + os.path.join(rocm, "lib")]

@@ -91,6 +91,12 @@ constexpr int SLOT_WORKERS = 4, SLOTS_PER_WORKER = 2;           // 16 MiB in all
 // 33 MB of bf16 no better either).
 constexpr size_t BANDS_TO_DEVICE_FROM = 48u << 20, BANDS_TO_HOST_FROM = 4u << 20;
 
+// A slot changes hands between the host and a kernel at an event of the kernel before, while kernels on other slots are still
+// running: coherent memory, stated here and not left to HIP_HOST_COHERENT, so that what a kernel has written is there once its
+// event has passed (it crosses no device cache that would have to be written back), and what the host has written before
+// a launch is read by it.
+constexpr unsigned SLOT_FLAGS = hipHostMallocPortable | hipHostMallocCoherent;
+
 // One set of slots per process, allocated on first use and given back with the runtime.  Whoever finds it taken (another
 // thread's transfer) goes without.
 std::mutex g_slots_guard;
@@ -117,7 +123,7 @@ bool through_slots(void *host, bool to_device, uint32_t batch, uint32_t h, size_
     if (hipStreamIsCapturing(stream, &capturing) != hipSuccess || capturing != hipStreamCaptureStatusNone) return false;
     std::unique_lock<std::mutex> taken(g_slots_guard, std::try_to_lock);
     if (!taken.owns_lock()) return false;
-    if (!g_slots && hipHostMalloc((void **)&g_slots, SLOT_BYTES * SLOT_WORKERS * SLOTS_PER_WORKER, hipHostMallocPortable) != hipSuccess) {
+    if (!g_slots && hipHostMalloc((void **)&g_slots, SLOT_BYTES * SLOT_WORKERS * SLOTS_PER_WORKER, SLOT_FLAGS) != hipSuccess) {
         (void)hipGetLastError();
         g_slots = nullptr;
         return false;
@@ -285,6 +291,17 @@ void require_rank4(const Dims &d, const char *what) {
 }
 
 }  // namespace
+
+#ifdef TTMI_TEST_HOOKS
+// Flags of the slots' allocation, as the runtime has them; nothing while there is none.
+std::optional<unsigned> test_slot_flags() {
+    std::lock_guard<std::mutex> lock(g_slots_guard);
+    unsigned flags = 0;
+    if (!g_slots) return std::nullopt;
+    hip_check(hipHostGetFlags(&flags, g_slots), "hipHostGetFlags");
+    return flags;
+}
+#endif
 
 void set_runtime(Runtime runtime) {
     if (!runtime.allocate) release_slots();

@@ -36,6 +36,9 @@ struct Runtime {
     std::function<bool()> gpu_available;
 };
 void set_runtime(Runtime runtime);
+#ifdef TTMI_TEST_HOOKS
+std::optional<unsigned> test_slot_flags();
+#endif
 
 struct Tensor {
     Buffer buffer;

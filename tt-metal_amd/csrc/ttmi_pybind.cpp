@@ -188,6 +188,9 @@ void bind_tensor_layer(py::module_ &m) {
 PYBIND11_MODULE(TTMI_PYBIND_NAME, m) {
     m.doc() = "Block-float tensors of tt-metal / TT-NN on MI355X: the host layer (Tensor and its operations) and the C ABI (include/ttmi.h)";
     bind_tensor_layer(m);
+#ifdef TTMI_TEST_HOOKS
+    m.def("test_slot_flags", &host::test_slot_flags);
+#endif
 
     m.attr("BFLOAT16") = (int)TTMI_BFLOAT16;
     m.attr("FLOAT32") = (int)TTMI_FLOAT32;
