@@ -163,6 +163,32 @@ SHAPES = [(1, 32, 4544, 18176), (1, 32, 18176, 4544), (1, 32, 4096, 6144), (1, 3
           (1, 32, 4096, 14336), (3, 24, 768, 160), (2, 40, 1024, 288), (1, 8, 32, 32), (1, 32, 64, 4096), (5, 100, 96, 2080)]
 
 
+def test_routes_with_scratch_of_the_library():
+    """Where calls without a workspace go that the library's scratch takes elsewhere than test_kernel_choice_by_shape says: the
+    kernel, the slices and rows that it sees (slices with common weights may become rows), and whether blocks are cut into k ranges."""
+    from ttmi import capi
+
+    L = _test_entries()
+    B8, B4, BF16 = capi.BFLOAT8_B, capi.BFLOAT4_B, capi.BFLOAT16
+    out = (ctypes.c_uint32 * 4)()
+    for args, want in [((1, 1, 1000, 14336, 4096, B4, BF16), (4, 1, 1000, 1)), ((1, 1, 2048, 4544, 18176, B8, BF16), (4, 1, 2048, 1)),
+                       ((1, 1, 1024, 4096, 4096, B8, BF16), (5, 1, 1024, 0)), ((8, 1, 384, 4096, 1024, B8, BF16), (5, 8, 384, 0)),
+                       # one round of the chip either way: no gain in joining the slices
+                       ((8, 1, 384, 1024, 4096, B8, BF16), (4, 8, 384, 0)), ((9, 1, 333, 1024, 4096, B8, BF16), (4, 1, 2997, 0)),
+                       ((5, 1, 150, 512, 2112, B8, BF16), (5, 1, 750, 0)), ((5, 5, 150, 512, 2112, B8, BF16), (3, 5, 150, 0)),
+                       # streamed and tiled shapes stay where they were
+                       ((2, 1, 32, 4096, 4096, B8, BF16), (2, 2, 32, 0)), ((1, 1, 200, 4096, 14336, B8, BF16), (2, 1, 200, 0)),
+                       ((12, 12, 384, 1024, 1024, B8, BF16), (3, 12, 384, 0))]:
+        L.ttmi_test_route(*args, out)
+        assert tuple(out) == want, args
+    # the public answer is that of weights per slice
+    P, plan = capi.lib(), (ctypes.c_uint32 * 4)()
+    for batch, m, k, n, fmt in [(1, 1000, 14336, 4096, B4), (1, 1024, 4096, 4096, B8), (5, 150, 512, 2112, B8), (8, 384, 1024, 4096, B8)]:
+        P.ttmi_matmul_bfp_plan(batch, m, k, n, BF16, fmt, BF16, plan)
+        L.ttmi_test_route(batch, batch, m, k, n, fmt, BF16, out)
+        assert plan[0] == out[0]
+
+
 def test_kernel_choice_by_shape():
     """Which kernel a GEMM goes to: one band streams in 128-column units, unless its 64-column groups are one workgroup per CU
     (200 to 256 of them) of at most 192 KiB of BFP4_B weights each and the output is not block-float — then the 64-column kernel

@@ -818,9 +818,11 @@ def test_every_kernel_packs_a_block_float_output_in_its_epilogue(oracle, out_fmt
     assert np.array_equal(got.cpu().numpy().view(np.uint32), host)
 
 
+@pytest.mark.parametrize("kernel", [None, "expanded"])
 @pytest.mark.parametrize("batch,b_batch,m,k,n", [(1, 1, 32, 64, 64), (1, 1, 32, 4544, 256), (2, 2, 40, 160, 96), (3, 1, 300, 96, 288), (1, 1, 512, 256, 544)])
-def test_bf16_weights(batch, b_batch, m, k, n):
-    """Two bf16 operands (ttmi_matmul_bf16): weights in TILE layout; against a float64 matmul of the same values with the bound of the block-float GEMMs; TILE and
+def test_bf16_weights(batch, b_batch, m, k, n, kernel, knobs):
+    """Two bf16 operands (ttmi_matmul_bf16), by the kernel that such shapes go to, which reads the weights where they lie, and by the one
+    behind a re-layout pass; weights in TILE layout; against a float64 matmul of the same values with the bound of the block-float GEMMs; TILE and
     row-major activations give the same bits; bias and activation; block-float output."""
     a_bits = workloads.activations_bf16(m, k, seed=500, batch=batch)
     w_bits = workloads.f32_to_bf16_bits_rne(workloads.weights_f32(k, n, seed=501, batch=b_batch))
@@ -828,6 +830,8 @@ def test_bf16_weights(batch, b_batch, m, k, n):
     w = workloads.bf16_bits_to_f32(w_bits).reshape(b_batch, k, n)
     a_dev = bf16_dev(a_bits).reshape(batch, m, k)
     w_tiles = capi.tilize(bf16_dev(w_bits).reshape(b_batch, k, n))
+    if kernel:
+        knobs("kernel", kernel)
     c = capi.matmul_bf16(a_dev, capi.ROW_MAJOR, w_tiles, batch, b_batch, m, k, n, out_dtype=torch.float32)
     for b in range(batch):
         check_against_reference(c[b].cpu().numpy(), a[b], w[b if b_batch > 1 else 0], k, bf16_out=False)
@@ -844,7 +848,11 @@ def test_bf16_weights(batch, b_batch, m, k, n):
     assert need == b_batch * (k // 32) * ((n // 32 + 1) // 2) * 4096
     ws = torch.full((need,), 0x5A, dtype=torch.uint8, device="cuda")
     again = capi.matmul_bf16(a_dev, capi.ROW_MAJOR, w_tiles, batch, b_batch, m, k, n, workspace=ws)
-    assert torch.equal(again.view(torch.int16), c16.view(torch.int16))
+    if kernel != "expanded" or k < 1024:
+        assert torch.equal(again.view(torch.int16), c16.view(torch.int16))
+    else:                        # k ranges, whose partial sums such a workspace has no room for: whole ranges there, another order of the sums
+        for b in range(batch):
+            check_against_reference(again[b].float().cpu().numpy(), a[b], w[b if b_batch > 1 else 0], k)
 
 
 GELU_KERNELS = ["stream", "wide", "tile", "expanded", "bf16 in place"]
@@ -954,9 +962,15 @@ def test_k_ranges_of_the_expanding_gemm(oracle, batch, m, k, n, fmt, knobs):
         assert np.array_equal(packed.cpu().numpy().view(np.uint32), host)
 
 
-@pytest.mark.parametrize("batch,m,k,n", [(8, 384, 1024, 4096), (5, 333, 512, 2112), (64, 32, 1024, 4096)])
-def test_slices_that_share_their_weights(batch, m, k, n):
+# slice by slice (the first two); as rows of one GEMM: of bf16 tiles, of 256 x 256 blocks, of such blocks with the last ones in k ranges,
+# rows that are no multiple of a tile among them, so that tiles and blocks begin in one slice and end in the next
+@pytest.mark.parametrize("batch,m,k,n,route", [(8, 384, 1024, 4096, (4, 8, 384, 0)), (5, 333, 512, 2112, (5, 5, 333, 0)), (64, 32, 1024, 4096, (5, 1, 2048, 0)), (5, 150, 512, 2112, (5, 1, 750, 0)),
+                                               (9, 333, 1024, 4096, (4, 1, 2997, 0)), (13, 333, 1024, 4096, (4, 1, 4329, 1))])
+def test_slices_that_share_their_weights(batch, m, k, n, route, test_library):
     """Slices with common weights, multiplied as the rows of one GEMM where that is better: float64, dense and tiles alike."""
+    out = (ctypes.c_uint32 * 4)()
+    test_library.ttmi_test_route(batch, 1, m, k, n, BFP8, capi.FLOAT32, out)
+    assert tuple(out) == route
     a = bf16_dev(workloads.activations_bf16(m, k, seed=530, batch=batch)).reshape(batch, m, k)
     words = capi.pack_tensor(BFP8, torch.from_numpy(workloads.weights_f32(k, n, seed=531)).cuda().reshape(1, k, n))
     w = capi.unpack_tensor(BFP8, words, (1, k, n))[0]

@@ -1210,8 +1210,10 @@ static Choice choose_kernel_own_scratch(uint32_t batch, uint32_t b_batch, uint32
 
 // Slices that share their weights are one GEMM of all their rows: [batch, m, k] lies in memory as [1, batch m, k] does, dense
 // or in whole tiles (TILE layouts have m % 32 == 0), and blocks of rows need not end with a slice.  Taken where the rows
-// together go to the expanding GEMM (or the one with smaller blocks) and that is the better one: 8 x [384, 1024] x [1024,
-// 4096] 39 us against 67 slice by slice (tiled).  Not for streamed shapes, whose slices share the weights through the caches:
+// together go to the expanding GEMM (or the one with smaller blocks) and that is the better one.  Measured, as rows / slice by
+// slice on the expanding GEMM / tiled / streamed: 9 x [333, 1024] x [1024, 4096] 37 / 59 / 63 / 59 us, 64 x [32, 1024] x [1024,
+// 4096] 32 / 124 / 117 / 44, 13 x [333, 1024] x [1024, 4096] 57 / 68 / 94 / 84.  Slices that need as many rounds of the chip either way
+// stay as they are: 8 x [384, 1024] x [1024, 4096] 43.0 / 43.2 (both on the expanding GEMM).  Not for streamed shapes, whose slices share the weights through the caches:
 // 2 x [32, 4096] x [4096, 4096] 13.6 against 10.2 us as they are.
 static bool fold_batch(const MatmulArgs &x, bool c_bfp) {
     const uint64_t rows = (uint64_t)x.batch * x.m;
@@ -1220,6 +1222,14 @@ static bool fold_batch(const MatmulArgs &x, bool c_bfp) {
     const Choice folded = choose_kernel_own_scratch(1, 1, (uint32_t)rows, x.k, x.n, x.b_fmt, c_bfp);
     if (folded.kernel != Kernel::Expanded && folded.kernel != Kernel::Direct) return false;
     return folded.us < choose_kernel_own_scratch(x.batch, 1, x.m, x.k, x.n, x.b_fmt, c_bfp).us;
+}
+
+// Where a call goes that has the library's scratch: the kernel, and the slices and rows that it sees.
+struct Route { Kernel kernel; uint32_t batch, m; };
+static Route own_scratch_route(const MatmulArgs &x, bool c_bfp) {
+    const bool folded = fold_batch(x, c_bfp);
+    const uint32_t batch = folded ? 1 : x.batch, m = folded ? x.batch * x.m : x.m;
+    return {choose_kernel_own_scratch(batch, x.b_batch, m, x.k, x.n, x.b_fmt, c_bfp).kernel, batch, m};
 }
 
 // Whether a call may go to `best` (as `batch` slices of `m` rows), which keeps expanded weights in scratch of the library's own,
@@ -1289,10 +1299,8 @@ int matmul_bfp(const MatmulArgs &asked, hipStream_t st) {
     Kernel kernel = choose_kernel(x.batch, x.m, x.k, x.n, x.b_fmt, c_bfp || a8);
     // (the workspace query answers for the slices as they are, so a caller's workspace serves those)
     if (!x.workspace && !x.no_alloc && !a8) {
-        const bool folded = fold_batch(x, c_bfp);
-        const uint32_t batch = folded ? 1 : x.batch, m = folded ? x.batch * x.m : x.m;
-        const Kernel best = choose_kernel_own_scratch(batch, x.b_batch, m, x.k, x.n, x.b_fmt, c_bfp).kernel;
-        if ((folded || best != kernel) && scratch_for(best, batch, m, kernel, x, st)) { kernel = best; x.batch = batch; x.m = m; }
+        const Route best = own_scratch_route(x, c_bfp);
+        if ((best.batch != x.batch || best.kernel != kernel) && scratch_for(best.kernel, best.batch, best.m, kernel, x, st)) { kernel = best.kernel; x.batch = best.batch; x.m = best.m; }
     }
     if (a8 && !matmul_takes_bfp_activations(x.batch, x.m, x.k, x.n, x.b_fmt))
         return fail(TTMI_ERR_UNSUPPORTED, "matmul: block-float activations are taken by the one-band streaming kernel only, which this shape does "
@@ -1414,6 +1422,15 @@ __attribute__((visibility("default"))) void ttmi_test_stream_decomposition(uint3
 // which kernel a shape goes to: 1 = 64-column streaming kernel, 2 = 128-column streaming kernel, 3 = tiled, 4 = expanded
 __attribute__((visibility("default"))) int ttmi_test_kernel_choice(uint32_t batch, uint32_t m, uint32_t k, uint32_t n, int b_fmt, int c_dtype) {
     return (int)ttmi::choose_kernel(batch, m, k, n, b_fmt, c_dtype == TTMI_BFLOAT8_B || c_dtype == TTMI_BFLOAT4_B);
+}
+// where a call with scratch of the library's own goes: out[0] the kernel (as above, 5 = bf16 tiles), out[1] the slices it sees (1: folded
+// into rows), out[2] the rows of each, out[3] whether the expanding GEMM cuts k ranges
+__attribute__((visibility("default"))) void ttmi_test_route(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, int b_fmt, int c_dtype, uint32_t out[4]) {
+    ttmi::MatmulArgs x{};
+    x.batch = batch; x.b_batch = b_batch; x.m = m; x.k = k; x.n = n; x.b_fmt = b_fmt;
+    const ttmi::Route r = ttmi::own_scratch_route(x, c_dtype == TTMI_BFLOAT8_B || c_dtype == TTMI_BFLOAT4_B);
+    out[0] = (uint32_t)r.kernel; out[1] = r.batch; out[2] = r.m;
+    out[3] = r.kernel == ttmi::Kernel::Expanded && ttmi::matmul_expanded_scratch_bytes(r.batch, b_batch, r.m, k, n) >= ttmi::matmul_expanded_workspace_bytes(b_batch, k, n) + (1u << 18);
 }
 __attribute__((visibility("default"))) void ttmi_test_wide_layout(int mantissa_bits, int lane, uint32_t out[16]) {
     if (mantissa_bits == 7) wide_layout_of<7>(lane, out); else wide_layout_of<3>(lane, out);
