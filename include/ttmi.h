@@ -167,7 +167,9 @@ TTMI_API size_t ttmi_matmul_bfp_workspace_bytes(uint32_t batch, uint32_t m, uint
  *            (up to 127 rows, and taller activations whose output has too few blocks to fill the chip) it holds partial
  *            sums of workgroups that share an output (a few MB); where they are expanded to bf16 first (from 512 rows
  *            on), the expanded weights (2 bytes per weight; the size query assumes every batch slice has weights of its
- *            own, a call with b_batch == 1 needs only one slice's worth)
+ *            own, a call with b_batch == 1 needs only one slice's worth).  With NULL more shapes are expanded, from 128 rows
+ *            on, and the library's buffer holds partial sums too (up to 64 MiB): the faster way for prompts of 128 rows and
+ *            more ([1000, 14336] x [14336, 4096] BFLOAT4_B 131 us, with a workspace 165)
  * fp32 accumulation throughout. */
 TTMI_API int ttmi_matmul_bfp(const void *a, int a_layout, const uint32_t *b, int b_fmt, uint32_t batch, uint32_t b_batch,
                     uint32_t m, uint32_t k, uint32_t n, const void *bias, int activation, void *c, int c_layout,
@@ -191,7 +193,9 @@ TTMI_API int ttmi_matmul_bfp_ab(const uint32_t *a, int a_fmt, const uint32_t *b,
                        size_t workspace_bytes, void *stream);
 
 /* Which kernel a block-float GEMM of this shape and these dtypes goes to, for whoever reads a profiler trace (no counterpart
- * in the reference, whose program factories log their choice; needs no GPU):
+ * in the reference, whose program factories log their choice; needs no GPU).  The answer is for a call without a workspace, outside
+ * a capture, whose slices have weights of their own (b_batch == batch): slices with common weights may run as the rows of one
+ * GEMM, and a call with a workspace, or ttmi_matmul_bfp_static, from 128 rows on takes kernels that need no more than that.
  *   out[0]  1 = 64-column streaming kernel, 2 = 128-column streaming kernel, 3 = fused tiled kernels, 4 = expansion + bf16 GEMM,
  *          5 = expansion to bf16 tiles + the GEMM of ttmi_matmul_bf16
  *   out[1]  k ranges per output (workgroups that share an output), streaming kernels only, else 0
@@ -224,8 +228,9 @@ TTMI_API int ttmi_matmul_bfp_gated(const void *a, int a_layout, const uint32_t *
                           int c_layout, int c_dtype, void *workspace, size_t workspace_bytes, void *stream);
 
 /* ttmi_matmul_bfp for callers that cannot allocate device memory: code under HIP graph capture, serving loops and
- * harnesses that forbid hipMalloc.  It has no counterpart in the reference.  Same arguments and results as
- * ttmi_matmul_bfp without the workspace pair; the scratch of the kernels lies in a static device array of
+ * harnesses that forbid hipMalloc.  It has no counterpart in the reference.  Same arguments as
+ * ttmi_matmul_bfp without the workspace pair, and its results but for the order of the fp32 sums, which from 128 rows on may be
+ * another (shapes that the library's own scratch takes to other kernels there); the scratch of the kernels lies in a static device array of
  * TTMI_STATIC_SCRATCH_BYTES (16 MiB) that every GPU the library runs on holds until the process ends, so the call
  * allocates nothing (no hipMalloc, hipFree or hipHostMalloc; the first call on a device resolves the array's address,
  * which is when the runtime places the array).  Shapes whose scratch does not fit

@@ -311,6 +311,13 @@ template <int WR, int WC, int RB, int CB, int STAGES> int launch_direct(DirectDe
 // 64 x 64 block 0.165 us alone and 0.143 us as one of many, 0.1 where the weights are few columns, which every L2 keeps
 // ([256, 8192] x [8192, 1024] 43 / 74 / 144, [4096, 4096] x [4096, 4096] 293 / 159 / 130, [3072, 4096] x [4096, 1024], block-float
 // weights, 44 / 47 / 53); a 256 x 256 block 0.72 us behind a pass over the weights and a second launch.
+// What the line at 1024 columns stands for is a jump of 64 blocks there, 128 ones do not have it.  BFLOAT8_B weights, the pass
+// over them included, 64 / 128 blocks at n = 768, 992, 1024, 1056, 1280, 1536, 2048:
+//   [2048, 4096] x [4096, n]  35/46 36/46 37/46 48/47 54/48 58/49 82/51
+//   [1024, 4096] x [4096, n]  31/47 32/47 30/46 34/47 34/47 37/48 40/49
+//   [3072, 4096] x [4096, n]  49/46 53/47 54/47 65/48 72/49 87/69 118/71
+//   [3072, 1024] x [1024, n]  17/18 19/19 20/19 22/20 23/21 27/25 33/26
+// so 0.1 is too little at 3072 rows (12 % lost up to 1024 columns on that box), and the estimate of 128 blocks too much from 1056 on.
 static double direct_us(uint32_t batch, uint32_t m, uint32_t k, uint32_t n, uint32_t *block) {
     const double steps = k / 32;
     auto blocks = [&](uint32_t edge) { return (double)batch * ((m + edge - 1) / edge) * ((n + edge - 1) / edge) / 256.0; };

@@ -88,8 +88,9 @@ void copy(Buffer &dst, const Buffer &src, size_t nbytes) {
 // ms; ttnn.from_torch 67 MB 2.59 -> 1.89 ms, 85 MB 3.27 -> 2.51 ms.
 constexpr size_t SLOT_BYTES = 2u << 20;
 constexpr int SLOT_WORKERS = 4, SLOTS_PER_WORKER = 2;           // 16 MiB in all
-// From where on: below, starting threads costs what it gains (from_torch: 4.2 MB 160 against 209 us, 16.8 MB 511 against 521,
-// 33 MB of bf16 no better either).
+// From where on.  To the host bands win from 4 MB.  To the device they do above 48 MiB; below, it is the box that decides: on one,
+// 4.2 MB took 160 us copied and 209 in bands, 16.8 MB 511 and 521; on another (4096 columns, copied / in bands) 7.9 MB 471 / 373,
+// 16.8 MB 878 / 718, 27.8 MB 1200 / 993, 43.5 MB 2840 / 1410, and of bf16 16.8 MB 792 / 710, 43.8 MB 2001 / 1471.
 constexpr size_t BANDS_TO_DEVICE_FROM = 48u << 20, BANDS_TO_HOST_FROM = 4u << 20;
 
 // A slot changes hands between the host and a kernel at an event of the kernel before, while kernels on other slots are still
