@@ -216,6 +216,16 @@ TTMI_API int ttmi_matmul_bf16(const void *a, int a_layout, const void *b, uint32
                      uint32_t n, const void *bias, int activation, void *c, int c_layout, int c_dtype, void *workspace,
                      size_t workspace_bytes, void *stream);
 
+/* ttmi_matmul_bfp, ttmi_matmul_bfp_ab or ttmi_matmul_bf16 (by a_dtype and b_dtype) with a bias that is read where it lies in TILE
+ * layout, as ttnn.linear holds it ([.., 32, N] with the values in row 0: ttnn/cpp/ttnn/operations/matmul.hpp:117-140), so that no
+ * untilize runs in front of the GEMM.  Bit for bit what those calls give for the row on its own.
+ *   a        TILE layout; a_dtype TTMI_BFLOAT16, or TTMI_BFLOAT8_B for shapes that ttmi_matmul_bfp_ab_supported() names
+ *   b        b_dtype TTMI_BFLOAT8_B | TTMI_BFLOAT4_B | TTMI_BFLOAT16 (the last with bf16 activations only)
+ *   bias     NULL or n / 32 bf16 tiles of 2048 bytes, of which row 0 counts
+ * The rest as there, without a workspace. */
+TTMI_API int ttmi_matmul_bias_tiles(const void *a, int a_dtype, const void *b, int b_dtype, uint32_t batch, uint32_t b_batch, uint32_t m,
+                           uint32_t k, uint32_t n, const void *bias, int activation, void *c, int c_layout, int c_dtype, void *stream);
+
 /* A gated pair of GEMMs in one launch:  C[b, m, n] = act(A . B_gate + bias) * (A . B_up), what a gated MLP issues as
  * ttnn.linear(x, w1, activation="silu"), ttnn.linear(x, w3) and ttnn.mul (models/demos/mistral7b/tt/mistral_mlp.py:43-82:
  * three device ops and two [m, n] intermediates there).  Both weight tensors have the shape, format and layout that

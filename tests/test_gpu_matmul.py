@@ -818,6 +818,30 @@ def test_every_kernel_packs_a_block_float_output_in_its_epilogue(oracle, out_fmt
     assert np.array_equal(got.cpu().numpy().view(np.uint32), host)
 
 
+@pytest.mark.parametrize("kernel", ["stream", "wide", "tile", "tile256", "tile4waves", "tile384", "expanded", "bf16 in place"])
+@pytest.mark.parametrize("batch,m,k,n", [(1, 32, 64, 32), (2, 96, 160, 288), (1, 384, 1024, 96)])
+def test_bias_in_tiles_is_the_row_on_its_own(oracle, kernel, batch, m, k, n, knobs):
+    """Every kernel reads a bias where it lies in TILE layout (row 0 of the tiles; the other rows hold NaN here, which must not
+    count) with the bits that the same n values in a row give: one tile, ragged column groups, shared outputs, each output type."""
+    block = {"tile256": 256, "tile4waves": 4, "tile384": 384}.get(kernel)
+    if block:
+        knobs("block", block)
+    knobs("kernel", "tile" if kernel.startswith("tile") else kernel)
+    words, _ = pack_weights(oracle, workloads.weights_f32(k, n, seed=421), BFP8)
+    a_tiles = capi.tilize(bf16_dev(workloads.activations_bf16(m, k, seed=420, batch=batch)).reshape(batch, m, k))
+    bias = bf16_dev(workloads.f32_to_bf16_bits_rne(workloads.normal_tensor((n,), seed=422)))
+    rows = torch.full((1, 32, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    rows[0, 0] = bias.reshape(n)
+    bias_tiles = capi.tilize(rows)
+    for out in ({}, {"out_dtype": torch.float32}) + (() if kernel == "stream" else ({"out_bfp": BFP8},)):      # the 64-column kernel packs no output
+        want = capi.matmul_bfp(a_tiles, capi.TILE, words, BFP8, batch, 1, m, k, n, c_layout=capi.TILE, bias=bias, activation=capi.ACT_SILU, **out)
+        got = torch.zeros_like(want)
+        c_dtype = BFP8 if "out_bfp" in out else capi.FLOAT32 if out else capi.BFLOAT16
+        capi.check(capi.lib().ttmi_matmul_bias_tiles(a_tiles.data_ptr(), capi.BFLOAT16, words.data_ptr(), BFP8, batch, 1, m, k, n, bias_tiles.data_ptr(),
+                                                     capi.ACT_SILU, got.data_ptr(), capi.TILE, c_dtype, torch.cuda.current_stream().cuda_stream))
+        assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+
+
 @pytest.mark.parametrize("kernel", [None, "expanded"])
 @pytest.mark.parametrize("batch,b_batch,m,k,n", [(1, 1, 32, 64, 64), (1, 1, 32, 4544, 256), (2, 2, 40, 160, 96), (3, 1, 300, 96, 288), (1, 1, 512, 256, 544)])
 def test_bf16_weights(batch, b_batch, m, k, n, kernel, knobs):

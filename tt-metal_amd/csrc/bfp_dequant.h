@@ -410,6 +410,13 @@ template <int W> __device__ __forceinline__ uint32_t to_code(uint32_t bits, uint
     return m ? (((bits >> 31) << W) | m) : 0u;
 }
 
+// Element of bias column `col`.  A bias in TILE layout is read where it lies (row 0 of its first row of tiles, four faces of 16 x 16
+// each): an untilize of its own in front of the GEMM is a launch that writes 32 rows for the one that counts.  A feed-forward
+// block of two biased GEMMs, [3072, 1024] x [1024, 4096] x [4096, 1024], BFLOAT8_B weights: 113.6 us with, 107.5 us without.
+__device__ __forceinline__ uint64_t bias_at(uint32_t col, int tiled) {
+    return tiled ? (uint64_t)(col >> 5) * 1024 + ((col >> 4) & 1) * 256 + (col & 15) : col;
+}
+
 // Epilogue of the tiled GEMM kernels for one wavefront: a 128-row x 64-column part of C (one 64-column weight group) whose
 // accumulators lie as v_mfma_f32_32x32x16 leaves them, with the column order of the weight expansion:
 //   acc[rb][cb][i] = row 32 rb + 8 (i / 4) + 4 kh + i % 4, column 32 t + 16 fc + 4 q + 2 half + cb of the 64, for lane
@@ -420,7 +427,7 @@ template <int W> __device__ __forceinline__ uint32_t to_code(uint32_t bits, uint
 // with 16 bytes per lane.  fp32 output is stored directly (8 bytes per lane).
 struct StoreTarget {
     uint8_t *c;              // output
-    const uint16_t *bias;    // bf16 [n] or null
+    const uint16_t *bias;    // bf16, n columns (bias_at), or null
     uint32_t m, n, nt;       // rows of a batch slice, columns, n / 32
     uint64_t slice;          // batch slice
     uint32_t row0;           // first row of the part
@@ -428,6 +435,7 @@ struct StoreTarget {
     float unscale;
     int c_tiled, c_f32;
     int c_bfp;               // 0, or the mantissa bits (7 | 3) of a block-float output (TILE layout)
+    int bias_tiled;          // bias is a row of tiles
 };
 
 template <int ACT, typename Acc, int RB>
@@ -442,7 +450,7 @@ __device__ __forceinline__ void store_wave_part(const Acc (&acc)[RB][2], const S
     float bias_v[2] = {0.f, 0.f};
     if (o.bias && lane_valid) {
 #pragma unroll
-        for (int cb = 0; cb < 2; ++cb) bias_v[cb] = __uint_as_float((uint32_t)o.bias[o.nt0 * 32 + col + cb] << 16);
+        for (int cb = 0; cb < 2; ++cb) bias_v[cb] = __uint_as_float((uint32_t)o.bias[bias_at(o.nt0 * 32 + col + cb, o.bias_tiled)] << 16);
     }
     const uint32_t mt = (o.m + 31) / 32;
     // Two loops and not a branch per element: the activations of neighbouring elements have to share a basic block to be

@@ -62,7 +62,8 @@ struct MatmulDev {
     const uint8_t *a;        // bf16
     const uint8_t *b;        // packed tiles
     const uint8_t *b2;       // gated form only: the second weight matrix (same shape and format), C = act(A.b) * (A.b2)
-    const uint16_t *bias;    // bf16 [n] or null
+    const uint16_t *bias;    // bf16, n columns (bias_at), or null
+    int bias_tiled;          // bias is a row of tiles
     uint8_t *c;              // output (bf16 or fp32)
     float *slots;            // 2 slots of 32x64 fp32 per workgroup, for outputs shared between workgroups (see SLOT_EMPTY)
     uint32_t *error;         // the device's error word (host memory): raised when a wait for partial sums gives up
@@ -444,7 +445,7 @@ __global__ __launch_bounds__(256, WGS_PER_CU) void matmul_stream_kernel(const Ma
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     float x = mine[r][j] * hidden_unscale;
-                    if (p.bias) x += __uint_as_float((uint32_t)p.bias[n_col + j] << 16);
+                    if (p.bias) x += __uint_as_float((uint32_t)p.bias[bias_at(n_col + j, p.bias_tiled)] << 16);
                     v[j] = apply_activation<ACT>(x);
                 }
                 uint64_t elem;   // element offset of the 4-column run in C
@@ -787,7 +788,7 @@ __global__ __launch_bounds__(256, NB == 2 ? 1 : WIDE_WGS_PER_CU) void matmul_wid
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             float x = sums[0][j] * (decode_unscale<W, MB>() * (A8 ? 0.015625f : 1.f));
-            if (p.bias) x += __uint_as_float((uint32_t)p.bias[n_col + j] << 16);
+            if (p.bias) x += __uint_as_float((uint32_t)p.bias[bias_at(n_col + j, p.bias_tiled)] << 16);
             v[j] = apply_activation<ACT>(x);
             if (NB == 2) v[j] *= sums[NB - 1][j] * decode_unscale<W, MB>();
         }
@@ -1049,7 +1050,7 @@ static uint32_t wide_grid_size(const Decomposition &d, bool in_xcds) {
 static int launch_streaming(const MatmulArgs &x, hipStream_t st, bool wide) {
     const Decomposition d = decompose(x.batch, x.m, x.k, x.n, wide, x.b2 != nullptr);
     MatmulDev p{};
-    p.a = (const uint8_t *)x.a; p.b = (const uint8_t *)x.b; p.b2 = (const uint8_t *)x.b2; p.bias = (const uint16_t *)x.bias; p.c = (uint8_t *)x.c;
+    p.a = (const uint8_t *)x.a; p.b = (const uint8_t *)x.b; p.b2 = (const uint8_t *)x.b2; p.bias = (const uint16_t *)x.bias; p.bias_tiled = x.bias_tiled; p.c = (uint8_t *)x.c;
     const bool gated = x.b2 != nullptr;
     if (gated && !wide) return fail(TTMI_ERR_UNSUPPORTED, "matmul: the gated form runs on the 128-column kernel only");
     const bool a8 = x.a_dtype == TTMI_BFLOAT8_B;

@@ -36,11 +36,11 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
 struct DirectDev {
     const uint8_t *a;        // bf16
     const uint8_t *b;        // bf16 tiles
-    const uint16_t *bias;    // bf16 [n] or null
+    const uint16_t *bias;    // bf16, n columns (bias_at), or null
     uint8_t *c;
     uint32_t b_batch, m, k, n;
     uint32_t kt, nt, mt, tiles_m, tiles_n, blocks, per_xcd;
-    int a_tiled, c_tiled, c_f32;
+    int a_tiled, c_tiled, c_f32, bias_tiled;
     int c_bfp;               // 0, or the mantissa bits (7 | 3) of a block-float output in TILE layout
     float unscale;           // common factor of the products: 1, or Wfmt::unscale for expanded block floats
 };
@@ -189,7 +189,7 @@ __global__ __launch_bounds__(256, 2) void matmul_direct_kernel(const DirectDev p
 #pragma unroll
                 for (int h = 0; h < 2; ++h) {
                     uint2 bias4 = make_uint2(0u, 0u);
-                    if (p.bias) __builtin_memcpy(&bias4, p.bias + col_tile * 32 + f * 16 + h * 8 + kh * 4, 8);      // a bias need not be aligned
+                    if (p.bias) __builtin_memcpy(&bias4, p.bias + bias_at(col_tile * 32 + f * 16 + h * 8 + kh * 4, p.bias_tiled), 8);      // a bias need not be aligned
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const uint32_t w = i < 2 ? bias4.x : bias4.y;
@@ -340,7 +340,7 @@ size_t matmul_direct_scratch_bytes(uint32_t b_batch, uint32_t k, uint32_t n) { r
 
 int matmul_bf16_direct(const MatmulArgs &x, hipStream_t st) {
     DirectDev p{};
-    p.a = (const uint8_t *)x.a; p.b = (const uint8_t *)x.b; p.bias = (const uint16_t *)x.bias; p.c = (uint8_t *)x.c;
+    p.a = (const uint8_t *)x.a; p.b = (const uint8_t *)x.b; p.bias = (const uint16_t *)x.bias; p.bias_tiled = x.bias_tiled; p.c = (uint8_t *)x.c;
     p.b_batch = x.b_batch; p.m = x.m; p.k = x.k; p.n = x.n;
     p.kt = x.k / 32; p.nt = x.n / 32; p.mt = (x.m + 31) / 32;
     p.a_tiled = x.a_layout == TTMI_TILE; p.c_tiled = x.c_layout == TTMI_TILE; p.c_f32 = x.c_dtype == TTMI_FLOAT32;

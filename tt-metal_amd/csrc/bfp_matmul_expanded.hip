@@ -134,7 +134,8 @@ __global__ __launch_bounds__(256) void relayout_bf16_kernel(const uint8_t *__res
 struct ExpandedDev {
     const uint8_t *a;        // bf16
     const uint8_t *w;        // expanded weights (workspace)
-    const uint16_t *bias;    // bf16 [n] or null
+    const uint16_t *bias;    // bf16, n columns (bias_at), or null
+    int bias_tiled;          // bias is a row of tiles
     uint8_t *c;
     uint32_t batch, b_batch, m, k, n;
     uint32_t kt, nt, groups, tiles_m, tiles_n;
@@ -308,7 +309,7 @@ __global__ __launch_bounds__(512, 1) void matmul_expanded_kernel(const ExpandedD
     }
 
     StoreTarget o;
-    o.c = p.c; o.bias = p.bias; o.m = p.m; o.n = p.n; o.nt = p.nt; o.slice = bb;
+    o.c = p.c; o.bias = p.bias; o.bias_tiled = p.bias_tiled; o.m = p.m; o.n = p.n; o.nt = p.nt; o.slice = bb;
     o.row0 = m0 + wr * 128; o.nt0 = (tn * 4 + wc) * 2;
     o.unscale = p.unscale; o.c_tiled = p.c_tiled; o.c_f32 = p.c_f32; o.c_bfp = p.c_bfp;
     store_wave_part<ACT>(acc, o, lds + wave * 16384, lane);
@@ -345,7 +346,7 @@ __global__ __launch_bounds__(256) void reduce_parts_kernel(const ExpandedDev p) 
         }
     }
     StoreTarget o;
-    o.c = p.c; o.bias = p.bias; o.m = p.m; o.n = p.n; o.nt = p.nt; o.slice = bb;
+    o.c = p.c; o.bias = p.bias; o.bias_tiled = p.bias_tiled; o.m = p.m; o.n = p.n; o.nt = p.nt; o.slice = bb;
     o.row0 = row0; o.nt0 = (tn * 4 + (w & 3)) * 2;
     o.unscale = p.unscale; o.c_tiled = p.c_tiled; o.c_f32 = p.c_f32; o.c_bfp = p.c_bfp;
     store_wave_part<ACT>(acc, o, lds + wave * 4096, lane);
@@ -410,7 +411,7 @@ template <int ACT> static void launch_expanded(const ExpandedDev &p, uint32_t bl
 // x.b: packed block-float tiles (x.b_fmt BFLOAT8_B | BFLOAT4_B) or bf16 tiles (x.b_fmt BFLOAT16)
 int matmul_bfp_expanded(const MatmulArgs &x, hipStream_t st) {
     ExpandedDev p{};
-    p.a = (const uint8_t *)x.a; p.bias = (const uint16_t *)x.bias; p.c = (uint8_t *)x.c;
+    p.a = (const uint8_t *)x.a; p.bias = (const uint16_t *)x.bias; p.bias_tiled = x.bias_tiled; p.c = (uint8_t *)x.c;
     p.batch = x.batch; p.b_batch = x.b_batch; p.m = x.m; p.k = x.k; p.n = x.n;
     p.kt = x.k / 32; p.nt = x.n / 32; p.groups = (p.nt + 1) / 2;
     p.tiles_m = (x.m + 255) / 256; p.tiles_n = (x.n + 255) / 256;

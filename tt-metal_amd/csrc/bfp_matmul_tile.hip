@@ -34,7 +34,8 @@ typedef __attribute__((__vector_size__(16 * sizeof(float)))) float f32x16;
 struct TileDev {
     const uint8_t *a;        // bf16
     const uint8_t *b;        // packed tiles
-    const uint16_t *bias;    // bf16 [n] or null
+    const uint16_t *bias;    // bf16, n columns (bias_at), or null
+    int bias_tiled;          // bias is a row of tiles
     uint8_t *c;              // output (bf16 or fp32)
     uint32_t batch, b_batch, m, k, n;
     uint32_t kt, nt, tiles_m, tiles_n;
@@ -257,7 +258,7 @@ __global__ __launch_bounds__(256, 1) void matmul_tile_kernel(const TileDev p) {
     __builtin_amdgcn_s_waitcnt(0xC07F);
     __builtin_amdgcn_s_barrier();
     StoreTarget o;
-    o.c = p.c; o.bias = p.bias; o.m = p.m; o.n = p.n; o.nt = p.nt; o.slice = bb;
+    o.c = p.c; o.bias = p.bias; o.bias_tiled = p.bias_tiled; o.m = p.m; o.n = p.n; o.nt = p.nt; o.slice = bb;
     o.row0 = m0; o.nt0 = nt0;
     o.unscale = F::unscale; o.c_tiled = p.c_tiled; o.c_f32 = p.c_f32; o.c_bfp = p.c_bfp;
     static_assert(MB == 4 && TILE_STAGES * STAGE_BYTES >= 4 * 16384, "the epilogue stages 128 rows x 64 columns per wavefront in the ring");
@@ -452,7 +453,7 @@ __global__ __launch_bounds__(512, 1) void matmul_tile8_kernel(const TileDev p) {
     __builtin_amdgcn_s_waitcnt(0xC07F);
     __builtin_amdgcn_s_barrier();
     StoreTarget o;
-    o.c = p.c; o.bias = p.bias; o.m = p.m; o.n = p.n; o.nt = p.nt; o.slice = bb;
+    o.c = p.c; o.bias = p.bias; o.bias_tiled = p.bias_tiled; o.m = p.m; o.n = p.n; o.nt = p.nt; o.slice = bb;
     o.row0 = m0 + wr * 32 * MB; o.nt0 = nt0;
     o.unscale = F::unscale; o.c_tiled = p.c_tiled; o.c_f32 = p.c_f32; o.c_bfp = p.c_bfp;
     static_assert(OPS_BASE + 2 * OPS_BYTES >= 8 * MB * 4096, "staging of the epilogue does not fit into LDS");
@@ -690,7 +691,7 @@ __global__ __launch_bounds__(64 * NW, 1) void matmul_tall_kernel(const TileDev p
     __builtin_amdgcn_s_waitcnt(0xC07F);
     __builtin_amdgcn_s_barrier();
     StoreTarget o;
-    o.c = p.c; o.bias = p.bias; o.m = p.m; o.n = p.n; o.nt = p.nt; o.slice = bb;
+    o.c = p.c; o.bias = p.bias; o.bias_tiled = p.bias_tiled; o.m = p.m; o.n = p.n; o.nt = p.nt; o.slice = bb;
     o.row0 = m0 + wave * 32; o.nt0 = nt0;
     o.unscale = F::unscale; o.c_tiled = p.c_tiled; o.c_f32 = p.c_f32; o.c_bfp = p.c_bfp;
     static_assert(LDS_BYTES >= NW * 4096, "staging of the epilogue does not fit into LDS");
@@ -734,7 +735,7 @@ static void launch_tile_act(const TileDev &p, int activation, uint32_t blocks, h
 
 int matmul_bfp_tiled(const MatmulArgs &x, hipStream_t st) {
     TileDev p{};
-    p.a = (const uint8_t *)x.a; p.b = (const uint8_t *)x.b; p.bias = (const uint16_t *)x.bias; p.c = (uint8_t *)x.c;
+    p.a = (const uint8_t *)x.a; p.b = (const uint8_t *)x.b; p.bias = (const uint16_t *)x.bias; p.bias_tiled = x.bias_tiled; p.c = (uint8_t *)x.c;
     p.batch = x.batch; p.b_batch = x.b_batch; p.m = x.m; p.k = x.k; p.n = x.n;
     p.kt = x.k / 32; p.nt = x.n / 32;
     p.a_tiled = x.a_layout == TTMI_TILE; p.c_tiled = x.c_layout == TTMI_TILE; p.c_f32 = x.c_dtype == TTMI_FLOAT32;

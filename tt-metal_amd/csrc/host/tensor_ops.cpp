@@ -564,21 +564,21 @@ Tensor matmul(const Tensor &a, const Tensor &b, bool bcast_batch, const Tensor *
     const int device = a.buffer.device;
     DeviceGuard guard(device);
     Buffer bias_row;
+    bool bias_tiles = false;
     if (bias) {
         if (!bias->on_device()) raise("TT_FATAL: bias must be on device");
         if (bias->padded.empty() || bias->padded.back() != n) raise("TT_FATAL: bias width must match the output width");
         if (bias->dtype != DataType::BFLOAT16 && !is_block_float(bias->dtype))
             raise(std::string("TT_FATAL: Unsupported data format for the bias: ") + name_of(bias->dtype));
-        // the bias is a [.., 32, N] tile row in the reference; its first row carries the values (matmul.hpp:117-140).  The GEMM
-        // reads n bf16 values: a row-major copy of that row.
+        // the bias is a [.., 32, N] tile row in the reference; its first row carries the values (matmul.hpp:117-140).  bf16 tiles
+        // the GEMM reads where they lie; for the rest it takes n bf16 values in a row.
         const uint32_t bh = bias->padded.size() > 1 ? bias->padded[bias->padded.size() - 2] : 1;
         if (is_block_float(bias->dtype)) {
             bias_row = allocate((size_t)bh * n * 2, device);
             check(ttmi_unpack_bfp_tiles_as_rowmajor((int)bias->dtype, (const uint32_t *)bias->buffer.data, 1, bh, n, bias_row.data, TTMI_BFLOAT16, stream_of(device)));
-        } else if (bias->layout == Layout::TILE) {
-            bias_row = relayout(false, bias->buffer, 2, {1, bh, n}, device);
         } else {
             bias_row = bias->buffer;
+            bias_tiles = bias->layout == Layout::TILE;
         }
     }
     const uint64_t a_elements = (uint64_t)batch_a * m * k, c_elements = (uint64_t)batch_a * m * n;
@@ -591,7 +591,10 @@ Tensor matmul(const Tensor &a, const Tensor &b, bool bcast_batch, const Tensor *
     const bool packed_out = is_block_float(out_dtype);
     const int c_layout = untilize_out ? TTMI_ROW_MAJOR : TTMI_TILE;                                     // bmm_op.cpp:1069
     Buffer c = allocate(packed_out ? storage_bytes(out_dtype, Layout::TILE, {batch_a, m, n}) : c_elements * 2, device);
-    if (b.dtype == DataType::BFLOAT16)      // two bf16 operands
+    if (bias_tiles)
+        check(ttmi_matmul_bias_tiles(a_tiles.data, a_in_kernel ? (int)a.dtype : TTMI_BFLOAT16, b.buffer.data, (int)b.dtype, batch_a, batch_b, m, k, n,
+                                     bias_row.data, activation, c.data, c_layout, packed_out ? (int)out_dtype : TTMI_BFLOAT16, stream_of(device)));
+    else if (b.dtype == DataType::BFLOAT16)      // two bf16 operands
         check(ttmi_matmul_bf16(a_tiles.data, TTMI_TILE, b.buffer.data, batch_a, batch_b, m, k, n, bias ? bias_row.data : nullptr, activation, c.data,
                                c_layout, packed_out ? (int)out_dtype : TTMI_BFLOAT16, nullptr, 0, stream_of(device)));
     else if (a_in_kernel)

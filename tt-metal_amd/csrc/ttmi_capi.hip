@@ -188,6 +188,17 @@ int ttmi_matmul_bfp_ab(const uint32_t *a, int a_fmt, const uint32_t *b, int b_fm
     return matmul_bfp(args, (hipStream_t)stream);
 }
 
+int ttmi_matmul_bias_tiles(const void *a, int a_dtype, const void *b, int b_dtype, uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k,
+                           uint32_t n, const void *bias, int activation, void *c, int c_layout, int c_dtype, void *stream) {
+    if (a_dtype != TTMI_BFLOAT16 && a_dtype != TTMI_BFLOAT8_B) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: activation dtype must be BFLOAT16 or BFLOAT8_B here, got %d", a_dtype);
+    if (a_dtype == TTMI_BFLOAT8_B && !is_bfp(b_dtype)) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: BFLOAT8_B activations need block-float weights, got dtype %d", b_dtype);
+    if (int rc = validate_matmul(a, TTMI_TILE, (const uint32_t *)b, b_dtype, batch, b_batch, m, k, n, activation, c, c_layout, c_dtype, true)) return rc;
+    MatmulArgs args{a, TTMI_TILE, (const uint32_t *)b, b_dtype, batch, b_batch, m, k, n, bias, activation, c, c_layout, c_dtype, nullptr, 0};
+    args.a_dtype = a_dtype;
+    args.bias_tiled = true;
+    return b_dtype == TTMI_BFLOAT16 ? matmul_bf16(args, (hipStream_t)stream) : matmul_bfp(args, (hipStream_t)stream);
+}
+
 size_t ttmi_matmul_bfp_gated_workspace_bytes(uint32_t batch, uint32_t m, uint32_t k, uint32_t n, int b_fmt) {
     (void)b_fmt;
     return matmul_gated_workspace_bytes(batch, m, k, n);

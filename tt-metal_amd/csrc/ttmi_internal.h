@@ -83,6 +83,7 @@ struct MatmulArgs {
     size_t workspace_empty_bytes = 0;            // this many leading bytes of the workspace are known to hold nothing but empty slots
     size_t *workspace_left_empty_bytes = nullptr;   // out: as above, after a launch that keeps its partial sums there (untouched otherwise)
     int a_dtype = TTMI_BFLOAT16;    // TTMI_BFLOAT8_B: `a` holds packed tiles (TILE layout), which the 128-column kernel expands itself
+    bool bias_tiled = false;        // `bias` is a row of bf16 tiles of which row 0 counts, not n values in a row
     bool no_alloc = false;          // the call may not allocate: `workspace` is all the scratch there is, its last 256 bytes stand
                                     // in for the error word when the device has none yet
 };
