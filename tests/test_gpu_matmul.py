@@ -842,6 +842,35 @@ def test_bias_in_tiles_is_the_row_on_its_own(oracle, kernel, batch, m, k, n, kno
         assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
 
 
+@pytest.mark.parametrize("fmt", [BFP8, BFP4, capi.BFLOAT16])
+@pytest.mark.parametrize("batch,m,k,n", [(8, 384, 64, 96), (2, 32, 96, 544), (5, 33, 64, 288), (3, 300, 1024, 64), (2, 384, 1024, 320)])
+def test_slices_with_common_weights_as_rows_of_the_expanding_gemm(oracle, fmt, batch, m, k, n, knobs):
+    """Slices joined into rows (fewer blocks, row blocks across slices, odd rows, k ranges cut in neither or in both) give the bits
+    that each slice gives on its own where no k range is cut, in every layout and output type that takes the shape."""
+    knobs("kernel", "expanded")
+    a = bf16_dev(workloads.activations_bf16(m, k, seed=430, batch=batch)).reshape(batch, m, k)
+    w = workloads.weights_f32(k, n, seed=431)
+    words = capi.tilize(dev(w).reshape(1, k, n).bfloat16()) if fmt == capi.BFLOAT16 else pack_weights(oracle, w, fmt)[0]
+    bias = bf16_dev(workloads.f32_to_bf16_bits_rne(workloads.normal_tensor((n,), seed=432)))
+
+    def product(x, layout, slices, **more):
+        if fmt == capi.BFLOAT16:
+            return capi.matmul_bf16(x, layout, words, slices, 1, m, k, n, bias=bias, **more)
+        return capi.matmul_bfp(x, layout, words, fmt, slices, 1, m, k, n, bias=bias, **more)
+
+    forms = [(capi.ROW_MAJOR, {}), (capi.ROW_MAJOR, {"out_dtype": torch.float32})]
+    if m % 32 == 0:
+        forms += [(capi.TILE, {"c_layout": capi.TILE})] + ([] if fmt == capi.BFLOAT16 else [(capi.TILE, {"c_layout": capi.TILE, "out_bfp": BFP8})])
+    for layout, more in forms:
+        operand = lambda x: capi.tilize(x) if layout == capi.TILE else x
+        got = product(operand(a), layout, batch, **more).reshape(-1)
+        want = torch.cat([product(operand(a[i:i + 1]), layout, 1, **more).reshape(-1) for i in range(batch)])
+        if k < 1024:                                         # one k range everywhere
+            assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+        elif "out_bfp" not in more:                          # sums in another order: 2K 2^-24 sum |a||w| < 1e-2 here, and a rounding to bf16
+            assert torch.allclose(got.float(), want.float(), rtol=2 ** -7, atol=1e-2)
+
+
 @pytest.mark.parametrize("kernel", [None, "expanded"])
 @pytest.mark.parametrize("batch,b_batch,m,k,n", [(1, 1, 32, 64, 64), (1, 1, 32, 4544, 256), (2, 2, 40, 160, 96), (3, 1, 300, 96, 288), (1, 1, 512, 256, 544)])
 def test_bf16_weights(batch, b_batch, m, k, n, kernel, knobs):

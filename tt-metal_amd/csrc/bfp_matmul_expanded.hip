@@ -403,13 +403,26 @@ int validate_expanded(const MatmulArgs &x) {
     return TTMI_OK;
 }
 
+// Slices with common weights run as the rows of one slice (the same memory: dense rows, or whole bands of tiles) where that takes
+// fewer blocks and as many rounds: 384 rows a slice pad to 512.  Only where neither way cuts k ranges, so that the scratch and
+// every sum are what they were.  8 x [384, 1024] x [1024, 4096], BFLOAT8_B weights, 192 blocks against 256 in one round:
+// 34.5 us against 42.8; with GELU and a block-float output 45.7 against 52.3.
+static bool rows_of_one_slice(const MatmulArgs &x) {
+    const uint64_t rows = (uint64_t)x.batch * x.m;
+    if (x.b_batch != 1 || x.batch == 1 || (rows + 31) / 32 * 64 * x.k > 0xffffffffull) return false;       // (validate_expanded: A of 4 GiB)
+    const ExpandedPlan slices = plan_expanded(x.batch, 1, x.m, x.k, x.n, 0, true), joined = plan_expanded(1, 1, (uint32_t)rows, x.k, x.n, 0, true);
+    return !slices.tail && !joined.tail && (rows + 255) / 256 < (uint64_t)x.batch * ((x.m + 255) / 256) && joined.us <= slices.us;
+}
+
 template <int ACT> static void launch_expanded(const ExpandedDev &p, uint32_t blocks, hipStream_t st) {
     hipLaunchKernelGGL((matmul_expanded_kernel<ACT>), dim3(blocks), dim3(512), 0, st, p);
     if (p.tail) hipLaunchKernelGGL((reduce_parts_kernel<ACT>), dim3(8 * p.tail * 8), dim3(256), 0, st, p);
 }
 
 // x.b: packed block-float tiles (x.b_fmt BFLOAT8_B | BFLOAT4_B) or bf16 tiles (x.b_fmt BFLOAT16)
-int matmul_bfp_expanded(const MatmulArgs &x, hipStream_t st) {
+int matmul_bfp_expanded(const MatmulArgs &asked, hipStream_t st) {
+    MatmulArgs x = asked;
+    if (rows_of_one_slice(x)) { x.m *= x.batch; x.batch = 1; }
     ExpandedDev p{};
     p.a = (const uint8_t *)x.a; p.bias = (const uint16_t *)x.bias; p.bias_tiled = x.bias_tiled; p.c = (uint8_t *)x.c;
     p.batch = x.batch; p.b_batch = x.b_batch; p.m = x.m; p.k = x.k; p.n = x.n;
