@@ -283,6 +283,24 @@ def test_strided_source_and_empty_inputs(oracle):
     assert capi.lib().ttmi_unpack_bfp_tiles_into_float_vec(BFP4, None, 0, 0, None, None) == 0
 
 
+@pytest.mark.parametrize("fmt", [3, 4])
+@pytest.mark.parametrize("n_tiles", [1, 3, 8, 13, 1025])
+def test_unpack_in_face_order_of_any_words(oracle, fmt, n_tiles):
+    """Face-ordered unpacking, chunks and typecast, of every exponent and code that words can hold (every other tile of ordinary rows, so
+    that wavefronts of both kinds occur), at tile counts that leave the last block partly empty: bit for bit the oracle's floats,
+    and as bf16 their upper halves (at most 7 significant bits)."""
+    rng = np.random.default_rng(n_tiles)
+    words = rng.integers(0, 2 ** 32, size=(n_tiles, capi.TILE_BYTES[fmt] // 4), dtype=np.uint32)
+    exponents = words[:, :16].view(np.uint8)
+    exponents[::2] = rng.integers(100, 140, size=exponents[::2].shape, dtype=np.uint8)
+    dev_words = torch.from_numpy(words.reshape(-1).view(np.int32)).cuda()
+    want = oracle.unpack_bfp_tiles_into_float_vec(fmt, words, False).view(np.uint32).reshape(-1)
+    for got in (capi.typecast_tiles(dev_words, fmt, capi.FLOAT32), capi.unpack_chunks(fmt, dev_words, row_major_output=False)):
+        assert np.array_equal(got.cpu().numpy().reshape(-1).view(np.uint32), want)
+    as_bf16 = capi.typecast_tiles(dev_words, fmt, capi.BFLOAT16).view(torch.int16).cpu().numpy().view(np.uint16)
+    assert np.array_equal(as_bf16.reshape(-1), (want >> 16).astype(np.uint16))
+
+
 @pytest.mark.parametrize("fmt", [capi.BFLOAT8_B, capi.BFLOAT4_B])
 def test_typecast_of_tile_ordered_tensors(oracle, fmt):
     """ttmi_typecast_tiles: block-float <-> bf16 / fp32 in tile order, one pass each way.  Towards block-float it is the host

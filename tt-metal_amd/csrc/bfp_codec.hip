@@ -348,11 +348,12 @@ __global__ __launch_bounds__(256) void pack_whole_kernel(const uint8_t *__restri
 }
 
 // ---------------------------------------------------------------------------------------------------------
-// unpack: the inverse walk.  ELEM is the destination element size (4 = fp32, 2 = bf16).
+// unpack: the inverse walk (face order has unpack_faces_kernel).  ELEM is the destination element size (4 = fp32, 2 = bf16).
 // ---------------------------------------------------------------------------------------------------------
 template <int W, int ELEM, int MODE, bool ALIGNED, int SHRINK = 0>
 __global__ __launch_bounds__(256) void unpack_kernel(const uint8_t *__restrict__ src, uint8_t *__restrict__ dst,
                                                      const CodecShape s) {
+    static_assert(MODE != SRC_TILE_FACES, "unpack_faces_kernel");
     using F = Fmt<W>;
     using I = Item<ELEM, SHRINK>;
     constexpr int TPB = I::TPB, EPL = I::EPL, ITS = I::ITS;
@@ -441,10 +442,52 @@ __global__ __launch_bounds__(256) void unpack_kernel(const uint8_t *__restrict__
             }
         } else {
             const uint64_t chunk = (tile0 + at.t) * 1024 * ELEM;
-            const int within = MODE == SRC_TILE_FACES ? (at.face * 256 + at.i * 16 + at.q * EPL)
-                                                      : (((at.face >> 1) * 16 + at.i) * 32 + (at.face & 1) * 16 + at.q * EPL);
+            const int within = ((at.face >> 1) * 16 + at.i) * 32 + (at.face & 1) * 16 + at.q * EPL;
             *reinterpret_cast<uint4 *>(dst + chunk + (uint64_t)within * ELEM) = v;
         }
+    }
+}
+
+// ---------------------------------------------------------------------------------------------------------
+// unpack in face order: codes and elements lie in the same order, so nothing has to change places and nothing goes through LDS.
+// 16 bytes of result per lane and piece, four pieces in flight; HBM-bound.  The arithmetic is unpack_kernel's.
+// ---------------------------------------------------------------------------------------------------------
+template <int W, int ELEM>
+__global__ __launch_bounds__(256) void unpack_faces_kernel(const uint8_t *__restrict__ src, uint4 *__restrict__ dst, uint64_t pieces) {
+    constexpr int EPL = 16 / ELEM, PIECES = 4, PER_TILE = 1024 / EPL, lane_bytes = EPL * (W + 1) / 8;
+    constexpr uint32_t all_mantissas = W == 7 ? 0x7f7f7f7fu : 0x77777777u;
+    const uint64_t first = (uint64_t)blockIdx.x * (256 * PIECES) + threadIdx.x;
+    uint32_t lo[PIECES], hi[PIECES], exps[PIECES];
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+        const uint64_t at = min(first + j * 256, pieces - 1);            // past the end: the last piece again, not stored
+        const uint32_t piece = (uint32_t)at % PER_TILE;
+        const uint8_t *tile = src + at / PER_TILE * Fmt<W>::tile_bytes, *codes = tile + 64 + piece * lane_bytes;
+        exps[j] = tile[piece * EPL / 16];
+        hi[j] = 0;
+        if (lane_bytes == 2) lo[j] = *reinterpret_cast<const uint16_t *>(codes);
+        else if (lane_bytes == 4) lo[j] = *reinterpret_cast<const uint32_t *>(codes);
+        else { const uint2 v = *reinterpret_cast<const uint2 *>(codes); lo[j] = v.x; hi[j] = v.y; }
+    }
+#pragma unroll
+    for (int j = 0; j < PIECES; ++j) {
+        const uint32_t shared = exps[j];
+        const bool tiny = shared < (uint32_t)W;
+        const bool odd_rows = __ballot((tiny && ((lo[j] | hi[j]) & all_mantissas) != 0) || shared >= 248u) != 0;
+        const float two_to = tiny ? 0.f : __uint_as_float((shared - (uint32_t)W + 1u) << 23);
+        uint32_t bits[EPL];
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) {
+            const int sh = (W + 1) * e;
+            const uint32_t field = sh < 32 ? (lo[j] >> sh) : (hi[j] >> (sh - 32));
+            if (!odd_rows) bits[e] = __float_as_uint((float)(field & ((1u << W) - 1u)) * two_to) | ((field << (31 - W)) & 0x80000000u);
+            else bits[e] = from_code<W>(field & ((2u << W) - 1u), shared);
+        }
+        uint4 v;
+        if (ELEM == 4) v = make_uint4(bits[0], bits[1], bits[2], bits[3]);
+        else v = make_uint4((bits[0] >> 16) | (bits[1 % EPL] & 0xffff0000u), (bits[2 % EPL] >> 16) | (bits[3 % EPL] & 0xffff0000u),
+                            (bits[4 % EPL] >> 16) | (bits[5 % EPL] & 0xffff0000u), (bits[6 % EPL] >> 16) | (bits[7 % EPL] & 0xffff0000u));
+        if (first + j * 256 < pieces) dst[first + j * 256] = v;
     }
 }
 
@@ -735,6 +778,13 @@ static void launch_unpack(bool aligned, const void *src, void *dst, const CodecS
     if (aligned) hipLaunchKernelGGL((unpack_kernel<W, ELEM, MODE, true, SHRINK>), dim3(blocks), dim3(256), 0, st, (const uint8_t *)src, (uint8_t *)dst, s);
     else hipLaunchKernelGGL((unpack_kernel<W, ELEM, MODE, false, SHRINK>), dim3(blocks), dim3(256), 0, st, (const uint8_t *)src, (uint8_t *)dst, s);
 }
+template <int W, int ELEM>
+static int launch_unpack_faces(const void *src, void *dst, uint64_t n_tiles, hipStream_t st) {
+    const uint64_t pieces = n_tiles * (64 * ELEM), blocks = (pieces + 1023) / 1024;
+    if (blocks > 0x7fffffffull) return fail(TTMI_ERR_INVALID_ARGUMENT, "unpack: too many tiles");
+    hipLaunchKernelGGL((unpack_faces_kernel<W, ELEM>), dim3((uint32_t)blocks), dim3(256), 0, st, (const uint8_t *)src, (uint4 *)dst, pieces);
+    return check_launch("unpack_faces_kernel");
+}
 // the tensor forms, with the block width chosen for the tensor (tensor_shape)
 template <int W, int ELEM>
 static void launch_pack_tensor(int shrink, bool aligned, const void *src, void *dst, const CodecShape &s, uint32_t blocks, hipStream_t st) {
@@ -797,10 +847,10 @@ int codec_unpack_chunks(int fmt, const uint32_t *words, size_t n_tiles, int row_
     if (blocks > 0x7fffffffull) return fail(TTMI_ERR_INVALID_ARGUMENT, "unpack: too many tiles");
     if (fmt == TTMI_BFLOAT8_B) {
         if (row_major_output) launch_unpack<7, 4, SRC_TILE_ROWMAJOR>(true, words, dst, s, (uint32_t)blocks, st);
-        else launch_unpack<7, 4, SRC_TILE_FACES>(true, words, dst, s, (uint32_t)blocks, st);
+        else return launch_unpack_faces<7, 4>(words, dst, n_tiles, st);
     } else {
         if (row_major_output) launch_unpack<3, 4, SRC_TILE_ROWMAJOR>(true, words, dst, s, (uint32_t)blocks, st);
-        else launch_unpack<3, 4, SRC_TILE_FACES>(true, words, dst, s, (uint32_t)blocks, st);
+        else return launch_unpack_faces<3, 4>(words, dst, n_tiles, st);
     }
     return check_launch("unpack_kernel");
 }
@@ -931,9 +981,8 @@ int codec_typecast_tiles(const void *src, int src_dtype, void *dst, int dst_dtyp
             else { if (elem == 4) launch_pack<3, 4, SRC_TILE_FACES>(true, src, dst, s, (uint32_t)blocks, st); else launch_pack<3, 2, SRC_TILE_FACES>(true, src, dst, s, (uint32_t)blocks, st); }
             return check_launch("pack_kernel");
         }
-        if (fmt == TTMI_BFLOAT8_B) { if (elem == 4) launch_unpack<7, 4, SRC_TILE_FACES>(true, src, dst, s, (uint32_t)blocks, st); else launch_unpack<7, 2, SRC_TILE_FACES>(true, src, dst, s, (uint32_t)blocks, st); }
-        else { if (elem == 4) launch_unpack<3, 4, SRC_TILE_FACES>(true, src, dst, s, (uint32_t)blocks, st); else launch_unpack<3, 2, SRC_TILE_FACES>(true, src, dst, s, (uint32_t)blocks, st); }
-        return check_launch("unpack_kernel");
+        if (fmt == TTMI_BFLOAT8_B) return elem == 4 ? launch_unpack_faces<7, 4>(src, dst, n_tiles, st) : launch_unpack_faces<7, 2>(src, dst, n_tiles, st);
+        return elem == 4 ? launch_unpack_faces<3, 4>(src, dst, n_tiles, st) : launch_unpack_faces<3, 2>(src, dst, n_tiles, st);
     }
     const uint64_t count = (uint64_t)n_tiles * 1024;
     const uint32_t blocks = (uint32_t)((count + 255) / 256 < 256 * 32 ? (count + 255) / 256 : 256 * 32);
