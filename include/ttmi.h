@@ -222,7 +222,8 @@ TTMI_API int ttmi_matmul_bf16(const void *a, int a_layout, const void *b, uint32
  *   a        TILE layout; a_dtype TTMI_BFLOAT16, or TTMI_BFLOAT8_B for shapes that ttmi_matmul_bfp_ab_supported() names
  *   b        b_dtype TTMI_BFLOAT8_B | TTMI_BFLOAT4_B | TTMI_BFLOAT16 (the last with bf16 activations only)
  *   bias     NULL or n / 32 bf16 tiles of 2048 bytes, of which row 0 counts
- * The rest as there, without a workspace. */
+ * The rest as there, without a workspace.  Shapes whose weights are streamed (up to 127 rows, and more where the output has few
+ * blocks: ttmi_matmul_bfp_plan) are refused with TTMI_ERR_UNSUPPORTED, before anything is launched. */
 TTMI_API int ttmi_matmul_bias_tiles(const void *a, int a_dtype, const void *b, int b_dtype, uint32_t batch, uint32_t b_batch, uint32_t m,
                            uint32_t k, uint32_t n, const void *bias, int activation, void *c, int c_layout, int c_dtype, void *stream);
 

@@ -62,8 +62,7 @@ struct MatmulDev {
     const uint8_t *a;        // bf16
     const uint8_t *b;        // packed tiles
     const uint8_t *b2;       // gated form only: the second weight matrix (same shape and format), C = act(A.b) * (A.b2)
-    const uint16_t *bias;    // bf16, n columns (bias_at), or null
-    int bias_tiled;          // bias is a row of tiles
+    const uint16_t *bias;    // bf16 [n] or null
     uint8_t *c;              // output (bf16 or fp32)
     float *slots;            // 2 slots of 32x64 fp32 per workgroup, for outputs shared between workgroups (see SLOT_EMPTY)
     uint32_t *error;         // the device's error word (host memory): raised when a wait for partial sums gives up
@@ -445,7 +444,7 @@ __global__ __launch_bounds__(256, WGS_PER_CU) void matmul_stream_kernel(const Ma
 #pragma unroll
                 for (int j = 0; j < 4; ++j) {
                     float x = mine[r][j] * hidden_unscale;
-                    if (p.bias) x += __uint_as_float((uint32_t)p.bias[bias_at(n_col + j, p.bias_tiled)] << 16);
+                    if (p.bias) x += __uint_as_float((uint32_t)p.bias[n_col + j] << 16);
                     v[j] = apply_activation<ACT>(x);
                 }
                 uint64_t elem;   // element offset of the 4-column run in C
@@ -788,7 +787,7 @@ __global__ __launch_bounds__(256, NB == 2 ? 1 : WIDE_WGS_PER_CU) void matmul_wid
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
             float x = sums[0][j] * (decode_unscale<W, MB>() * (A8 ? 0.015625f : 1.f));
-            if (p.bias) x += __uint_as_float((uint32_t)p.bias[bias_at(n_col + j, p.bias_tiled)] << 16);
+            if (p.bias) x += __uint_as_float((uint32_t)p.bias[n_col + j] << 16);
             v[j] = apply_activation<ACT>(x);
             if (NB == 2) v[j] *= sums[NB - 1][j] * decode_unscale<W, MB>();
         }
@@ -1050,7 +1049,7 @@ static uint32_t wide_grid_size(const Decomposition &d, bool in_xcds) {
 static int launch_streaming(const MatmulArgs &x, hipStream_t st, bool wide) {
     const Decomposition d = decompose(x.batch, x.m, x.k, x.n, wide, x.b2 != nullptr);
     MatmulDev p{};
-    p.a = (const uint8_t *)x.a; p.b = (const uint8_t *)x.b; p.b2 = (const uint8_t *)x.b2; p.bias = (const uint16_t *)x.bias; p.bias_tiled = x.bias_tiled; p.c = (uint8_t *)x.c;
+    p.a = (const uint8_t *)x.a; p.b = (const uint8_t *)x.b; p.b2 = (const uint8_t *)x.b2; p.bias = (const uint16_t *)x.bias; p.c = (uint8_t *)x.c;
     const bool gated = x.b2 != nullptr;
     if (gated && !wide) return fail(TTMI_ERR_UNSUPPORTED, "matmul: the gated form runs on the 128-column kernel only");
     const bool a8 = x.a_dtype == TTMI_BFLOAT8_B;
@@ -1214,7 +1213,7 @@ static Choice choose_kernel_own_scratch(uint32_t batch, uint32_t b_batch, uint32
 // together go to the expanding GEMM (or the one with smaller blocks) and that is the better one.  Measured, as rows / slice by
 // slice on the expanding GEMM / tiled / streamed: 9 x [333, 1024] x [1024, 4096] 37 / 59 / 63 / 59 us, 64 x [32, 1024] x [1024,
 // 4096] 32 / 124 / 117 / 44, 13 x [333, 1024] x [1024, 4096] 57 / 68 / 94 / 84.  Slices that need as many rounds of the chip either way
-// stay as they are: 8 x [384, 1024] x [1024, 4096] 43.0 / 43.2 (both on the expanding GEMM).  Not for streamed shapes, whose slices share the weights through the caches:
+// keep their route; the expanding GEMM joins those by itself where that saves blocks (rows_of_one_slice).  Not for streamed shapes, whose slices share the weights through the caches:
 // 2 x [32, 4096] x [4096, 4096] 13.6 against 10.2 us as they are.
 static bool fold_batch(const MatmulArgs &x, bool c_bfp) {
     const uint64_t rows = (uint64_t)x.batch * x.m;
@@ -1306,6 +1305,10 @@ int matmul_bfp(const MatmulArgs &asked, hipStream_t st) {
     if (a8 && !matmul_takes_bfp_activations(x.batch, x.m, x.k, x.n, x.b_fmt))
         return fail(TTMI_ERR_UNSUPPORTED, "matmul: block-float activations are taken by the one-band streaming kernel only, which this shape does "
                     "not go to (ttmi_matmul_bfp_ab_supported): expand them with ttmi_typecast_tiles first");
+    // The streaming kernels take a bias as a row only: with the index of a tile in their epilogues [96, 4544] x [4544, 4672], which has no
+    // bias at all, took 17.7 us instead of 16.1.
+    if (x.bias_tiled && x.bias && (kernel == Kernel::Wide || kernel == Kernel::Stream))
+        return fail(TTMI_ERR_UNSUPPORTED, "matmul: the streaming kernels take no bias in tiles: untilize its first row first");
     switch (kernel) {
         case Kernel::Direct: return matmul_bf16_direct(x, st);
         case Kernel::Expanded: return matmul_bfp_expanded(x, st);

@@ -571,7 +571,7 @@ Tensor matmul(const Tensor &a, const Tensor &b, bool bcast_batch, const Tensor *
         if (bias->dtype != DataType::BFLOAT16 && !is_block_float(bias->dtype))
             raise(std::string("TT_FATAL: Unsupported data format for the bias: ") + name_of(bias->dtype));
         // the bias is a [.., 32, N] tile row in the reference; its first row carries the values (matmul.hpp:117-140).  bf16 tiles
-        // the GEMM reads where they lie; for the rest it takes n bf16 values in a row.
+        // most GEMMs read where they lie; else they take n bf16 values in a row.
         const uint32_t bh = bias->padded.size() > 1 ? bias->padded[bias->padded.size() - 2] : 1;
         if (is_block_float(bias->dtype)) {
             bias_row = allocate((size_t)bh * n * 2, device);
@@ -591,10 +591,16 @@ Tensor matmul(const Tensor &a, const Tensor &b, bool bcast_batch, const Tensor *
     const bool packed_out = is_block_float(out_dtype);
     const int c_layout = untilize_out ? TTMI_ROW_MAJOR : TTMI_TILE;                                     // bmm_op.cpp:1069
     Buffer c = allocate(packed_out ? storage_bytes(out_dtype, Layout::TILE, {batch_a, m, n}) : c_elements * 2, device);
-    if (bias_tiles)
-        check(ttmi_matmul_bias_tiles(a_tiles.data, a_in_kernel ? (int)a.dtype : TTMI_BFLOAT16, b.buffer.data, (int)b.dtype, batch_a, batch_b, m, k, n,
-                                     bias_row.data, activation, c.data, c_layout, packed_out ? (int)out_dtype : TTMI_BFLOAT16, stream_of(device)));
-    else if (b.dtype == DataType::BFLOAT16)      // two bf16 operands
+    bool done = false;
+    if (bias_tiles) {
+        const int rc = ttmi_matmul_bias_tiles(a_tiles.data, a_in_kernel ? (int)a.dtype : TTMI_BFLOAT16, b.buffer.data, (int)b.dtype, batch_a, batch_b, m, k, n,
+                                              bias_row.data, activation, c.data, c_layout, packed_out ? (int)out_dtype : TTMI_BFLOAT16, stream_of(device));
+        done = rc != TTMI_ERR_UNSUPPORTED;
+        if (done) check(rc);
+        else bias_row = relayout(false, bias->buffer, 2, {1, bias->padded.size() > 1 ? bias->padded[bias->padded.size() - 2] : 1, n}, device);      // a kernel that takes a row
+    }
+    if (done) {
+    } else if (b.dtype == DataType::BFLOAT16)      // two bf16 operands
         check(ttmi_matmul_bf16(a_tiles.data, TTMI_TILE, b.buffer.data, batch_a, batch_b, m, k, n, bias ? bias_row.data : nullptr, activation, c.data,
                                c_layout, packed_out ? (int)out_dtype : TTMI_BFLOAT16, nullptr, 0, stream_of(device)));
     else if (a_in_kernel)
