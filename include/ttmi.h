@@ -216,14 +216,19 @@ TTMI_API int ttmi_matmul_bf16(const void *a, int a_layout, const void *b, uint32
                      uint32_t n, const void *bias, int activation, void *c, int c_layout, int c_dtype, void *workspace,
                      size_t workspace_bytes, void *stream);
 
+/* 1 where the calls below take a bias in TILE layout for these sizes and types (bf16 activations), 0 where the weights are streamed: those
+ * kernels read a bias as n values in a row only, so the caller untilizes its row 0 first and calls ttmi_matmul_bfp.  Needs no GPU, and answers for a
+ * call that gets the scratch it asks for (see there). */
+TTMI_API int ttmi_matmul_bias_tiles_supported(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, int b_dtype, int c_dtype);
+
 /* ttmi_matmul_bfp, ttmi_matmul_bfp_ab or ttmi_matmul_bf16 (by a_dtype and b_dtype) with a bias that is read where it lies in TILE
  * layout, as ttnn.linear holds it ([.., 32, N] with the values in row 0: ttnn/cpp/ttnn/operations/matmul.hpp:117-140), so that no
  * untilize runs in front of the GEMM.  Bit for bit what those calls give for the row on its own.
  *   a        TILE layout; a_dtype TTMI_BFLOAT16, or TTMI_BFLOAT8_B for shapes that ttmi_matmul_bfp_ab_supported() names
  *   b        b_dtype TTMI_BFLOAT8_B | TTMI_BFLOAT4_B | TTMI_BFLOAT16 (the last with bf16 activations only)
  *   bias     NULL or n / 32 bf16 tiles of 2048 bytes, of which row 0 counts
- * The rest as there, without a workspace.  Shapes whose weights are streamed (up to 127 rows, and more where the output has few
- * blocks: ttmi_matmul_bfp_plan) are refused with TTMI_ERR_UNSUPPORTED, before anything is launched. */
+ * The rest as there, without a workspace.  Shapes whose weights are streamed (ttmi_matmul_bias_tiles_supported: 0), and those that are
+ * for want of scratch (no device memory, or a graph capture that finds none), are refused with TTMI_ERR_UNSUPPORTED, before anything is launched. */
 TTMI_API int ttmi_matmul_bias_tiles(const void *a, int a_dtype, const void *b, int b_dtype, uint32_t batch, uint32_t b_batch, uint32_t m,
                            uint32_t k, uint32_t n, const void *bias, int activation, void *c, int c_layout, int c_dtype, void *stream);
 

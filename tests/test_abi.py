@@ -189,6 +189,32 @@ def test_routes_with_scratch_of_the_library():
         assert plan[0] == out[0]
 
 
+def test_bias_in_tiles_is_promised_by_the_route():
+    """ttmi_matmul_bias_tiles_supported: 1 exactly where the route with the library's scratch is a kernel that does not stream (one to
+    four bands, streamed prompts, folded slices, weights per slice, block-float outputs), always for bf16 weights, 0 for what no GEMM takes."""
+    from ttmi import capi
+
+    L = _test_entries()
+    supported = capi.lib().ttmi_matmul_bias_tiles_supported
+    B8, B4, BF16 = capi.BFLOAT8_B, capi.BFLOAT4_B, capi.BFLOAT16
+    out, seen = (ctypes.c_uint32 * 4)(), set()
+    for batch in (1, 8, 64):
+        for b_batch in {1, batch}:
+            for m in (1, 32, 64, 96, 128, 200, 384, 1000, 2048):
+                for k, n in [(64, 32), (1024, 4096), (4096, 1024), (4544, 4672), (4096, 14336), (14336, 4096)]:
+                    for fmt in (B8, B4):
+                        for c_dtype in (BF16, B8):
+                            L.ttmi_test_route(batch, b_batch, m, k, n, fmt, c_dtype, out)
+                            got = supported(batch, b_batch, m, k, n, fmt, c_dtype)
+                            assert got == (out[0] not in (1, 2)), (batch, b_batch, m, k, n, fmt, c_dtype)
+                            seen.add(got)
+                    assert supported(batch, b_batch, m, k, n, BF16, BF16) == 1
+    assert seen == {0, 1}
+    for args in [(0, 1, 384, 64, 64, B8, BF16), (1, 1, 0, 64, 64, BF16, BF16), (1, 1, 384, 40, 64, BF16, BF16), (1, 1, 2048, 4096, 14340, B8, BF16),
+                 (1, 1, 2048, 4096, 14336, capi.FLOAT32, BF16)]:
+        assert supported(*args) == 0
+
+
 def test_kernel_choice_by_shape():
     """Which kernel a GEMM goes to: one band streams in 128-column units, unless its 64-column groups are one workgroup per CU
     (200 to 256 of them) of at most 192 KiB of BFP4_B weights each and the output is not block-float — then the 64-column kernel

@@ -130,6 +130,52 @@ def test_linear_bias_activation(device, activation, use_bias):
     assert np.corrcoef(got.numpy().ravel(), ref.numpy().ravel())[0, 1] >= 0.9999
 
 
+def _same_bias(n, device):
+    """Values that a block-float tensor holds exactly, as one (which is always unpacked into a row) and in bf16 tiles."""
+    import ttnn
+
+    packed = ttnn.from_torch(torch.randn((1, n)), layout=ttnn.TILE_LAYOUT, device=device, dtype=ttnn.bfloat8_b)
+    return packed, ttnn.from_torch(ttnn.to_torch(packed).bfloat16(), layout=ttnn.TILE_LAYOUT, device=device)
+
+
+@pytest.mark.parametrize("m,k,n,a_type,b_type", [
+    (32, 64, 32, "bfloat16", "bfloat8_b"), (32, 1024, 4096, "bfloat8_b", "bfloat8_b"), (96, 256, 512, "bfloat16", "bfloat4_b"), (224, 4096, 1024, "bfloat16", "bfloat8_b"),      # streamed
+    (512, 1024, 4096, "bfloat16", "bfloat8_b"), (384, 1024, 4096, "bfloat8_b", "bfloat4_b"), (64, 96, 160, "bfloat16", "bfloat16")])
+def test_bias_in_tiles_by_one_call(device, m, k, n, a_type, b_type):
+    """A bias in TILE layout: the bits of the same values in a row, whichever kernel the shape goes to, and no call on the way is
+    refused (the last error of this thread stays what it was)."""
+    import ttnn
+    from ttmi import capi
+
+    torch.manual_seed(4)
+    a = ttnn.from_torch(torch.randn((1, m, k), dtype=torch.bfloat16), layout=ttnn.TILE_LAYOUT, device=device, dtype=getattr(ttnn, a_type))
+    b = ttnn.from_torch(torch.randn((k, n), dtype=torch.bfloat16) * 0.1, layout=ttnn.TILE_LAYOUT, device=device, dtype=getattr(ttnn, b_type))
+    row, tiles = _same_bias(n, device)
+    assert capi.lib().ttmi_tilize(None, 3, 1, 32, 32, None, None) != 0
+    before = capi.lib().ttmi_last_error()
+    got = ttnn.linear(a, b, bias=tiles, activation="silu", dtype=ttnn.bfloat16)
+    assert capi.lib().ttmi_last_error() == before
+    assert torch.equal(ttnn.to_torch(got), ttnn.to_torch(ttnn.linear(a, b, bias=row, activation="silu", dtype=ttnn.bfloat16)))
+
+
+def test_bias_in_tiles_without_memory_for_scratch(knobs):
+    """A shape that reads the bias in tiles, on a device without memory for the expanded weights: the weights are streamed, with a bias in a row."""
+    import ttnn
+    from ttmi import capi
+
+    m, k, n = 1024, 4096, 4096
+    assert capi.lib().ttmi_matmul_bias_tiles_supported(1, 1, m, k, n, capi.BFLOAT8_B, capi.BFLOAT16) == 1
+    device = ttnn.open_device(0)
+    torch.manual_seed(5)
+    a = ttnn.from_torch(torch.randn((1, m, k), dtype=torch.bfloat16), layout=ttnn.TILE_LAYOUT, device=device)
+    b = ttnn.from_torch(torch.randn((k, n), dtype=torch.bfloat16) * 0.1, layout=ttnn.TILE_LAYOUT, device=device, dtype=ttnn.bfloat8_b)
+    row, tiles = _same_bias(n, device)
+    torch.cuda.synchronize()
+    capi.release_scratch()
+    knobs("scratch_limit", k * n * 2 - 1)
+    assert torch.equal(ttnn.to_torch(ttnn.linear(a, b, bias=tiles)), ttnn.to_torch(ttnn.linear(a, b, bias=row)))
+
+
 def test_matmul_errors(device):
     import ttnn
 

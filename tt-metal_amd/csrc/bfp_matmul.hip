@@ -1288,6 +1288,15 @@ bool matmul_takes_bfp_activations(uint32_t batch, uint32_t m, uint32_t k, uint32
     return batch && m == 32 && k && n && choose_kernel(batch, m, k, n, b_fmt, true) == Kernel::Wide;
 }
 
+bool matmul_takes_bias_tiles(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, int b_fmt, bool c_bfp) {
+    if (!batch || !m || !k || !n) return false;
+    if (b_fmt == TTMI_BFLOAT16) return true;      // neither of the kernels of two bf16 operands streams
+    MatmulArgs x{};
+    x.batch = batch; x.b_batch = b_batch; x.m = m; x.k = k; x.n = n; x.b_fmt = b_fmt;
+    const Kernel kernel = own_scratch_route(x, c_bfp).kernel;
+    return kernel != Kernel::Wide && kernel != Kernel::Stream;
+}
+
 int matmul_bfp(const MatmulArgs &asked, hipStream_t st) {
     MatmulArgs x = asked;
     // what an earlier launch on this device has reported (a wait for partial sums that gave up) surfaces here

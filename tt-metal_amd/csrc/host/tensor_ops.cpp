@@ -563,54 +563,57 @@ Tensor matmul(const Tensor &a, const Tensor &b, bool bcast_batch, const Tensor *
         raise("TT_FATAL: this->output_dtype == DataType::BFLOAT16 (untilize_out writes a ROW_MAJOR output, which a block-float tensor cannot be)");
     const int device = a.buffer.device;
     DeviceGuard guard(device);
+    const bool packed_out = is_block_float(out_dtype);
+    const int c_dtype = packed_out ? (int)out_dtype : TTMI_BFLOAT16;
+    // block-float activations are expanded (exactly) to bf16 tiles by one kernel in front of the GEMM, unless the shape goes to the kernel
+    // that streams the weights, which takes BFLOAT8_B activations as they are
+    const bool a_in_kernel = is_block_float(b.dtype) && ttmi_matmul_bfp_ab_supported(batch_a, m, k, n, (int)a.dtype, (int)b.dtype);
     Buffer bias_row;
     bool bias_tiles = false;
+    const uint32_t bh = bias && bias->padded.size() > 1 ? bias->padded[bias->padded.size() - 2] : 1;
     if (bias) {
         if (!bias->on_device()) raise("TT_FATAL: bias must be on device");
         if (bias->padded.empty() || bias->padded.back() != n) raise("TT_FATAL: bias width must match the output width");
         if (bias->dtype != DataType::BFLOAT16 && !is_block_float(bias->dtype))
             raise(std::string("TT_FATAL: Unsupported data format for the bias: ") + name_of(bias->dtype));
         // the bias is a [.., 32, N] tile row in the reference; its first row carries the values (matmul.hpp:117-140).  bf16 tiles
-        // most GEMMs read where they lie; else they take n bf16 values in a row.
-        const uint32_t bh = bias->padded.size() > 1 ? bias->padded[bias->padded.size() - 2] : 1;
+        // the GEMMs that do not stream the weights read where they lie; the others take n bf16 values in a row.  Which it is
+        // the route says beforehand: [32, 4096] x [4096, 4096] is bound by its submission, and asking by a call that is
+        // refused took 17.1 us where the untilize at once takes 15.0.
         if (is_block_float(bias->dtype)) {
             bias_row = allocate((size_t)bh * n * 2, device);
             check(ttmi_unpack_bfp_tiles_as_rowmajor((int)bias->dtype, (const uint32_t *)bias->buffer.data, 1, bh, n, bias_row.data, TTMI_BFLOAT16, stream_of(device)));
         } else {
-            bias_row = bias->buffer;
-            bias_tiles = bias->layout == Layout::TILE;
+            bias_tiles = bias->layout == Layout::TILE && !a_in_kernel && ttmi_matmul_bias_tiles_supported(batch_a, batch_b, m, k, n, (int)b.dtype, c_dtype);
+            bias_row = bias->layout == Layout::TILE && !bias_tiles ? relayout(false, bias->buffer, 2, {1, bh, n}, device) : bias->buffer;
         }
     }
     const uint64_t a_elements = (uint64_t)batch_a * m * k, c_elements = (uint64_t)batch_a * m * n;
-    // block-float activations are expanded (exactly) to bf16 tiles by one kernel in front of the GEMM; a block-float output is
-    // packed by the GEMM itself, in its epilogue (the host packers' arithmetic on the bf16-rounded sums: parity with the
-    // Tensix packer unpinned)
-    // ... unless the shape goes to the kernel that streams the weights, which takes BFLOAT8_B activations as they are
-    const bool a_in_kernel = is_block_float(b.dtype) && ttmi_matmul_bfp_ab_supported(batch_a, m, k, n, (int)a.dtype, (int)b.dtype);
+    // a block-float output is packed by the GEMM itself, in its epilogue (the host packers' arithmetic on the bf16-rounded sums:
+    // parity with the Tensix packer unpinned)
     Buffer a_tiles = is_block_float(a.dtype) && !a_in_kernel ? typecast_tiles(a.buffer, a.dtype, DataType::BFLOAT16, a_elements, device) : a.buffer;
-    const bool packed_out = is_block_float(out_dtype);
     const int c_layout = untilize_out ? TTMI_ROW_MAJOR : TTMI_TILE;                                     // bmm_op.cpp:1069
     Buffer c = allocate(packed_out ? storage_bytes(out_dtype, Layout::TILE, {batch_a, m, n}) : c_elements * 2, device);
-    bool done = false;
+    int rc = TTMI_ERR_UNSUPPORTED;
     if (bias_tiles) {
-        const int rc = ttmi_matmul_bias_tiles(a_tiles.data, a_in_kernel ? (int)a.dtype : TTMI_BFLOAT16, b.buffer.data, (int)b.dtype, batch_a, batch_b, m, k, n,
-                                              bias_row.data, activation, c.data, c_layout, packed_out ? (int)out_dtype : TTMI_BFLOAT16, stream_of(device));
-        done = rc != TTMI_ERR_UNSUPPORTED;
-        if (done) check(rc);
-        else bias_row = relayout(false, bias->buffer, 2, {1, bias->padded.size() > 1 ? bias->padded[bias->padded.size() - 2] : 1, n}, device);      // a kernel that takes a row
+        rc = ttmi_matmul_bias_tiles(a_tiles.data, TTMI_BFLOAT16, b.buffer.data, (int)b.dtype, batch_a, batch_b, m, k, n, bias_row.data, activation, c.data,
+                                    c_layout, c_dtype, stream_of(device));
+        // refused: there is no scratch for the route, and the GEMM streams the weights after all
+        if (rc == TTMI_ERR_UNSUPPORTED) bias_row = relayout(false, bias->buffer, 2, {1, bh, n}, device);
     }
-    if (done) {
-    } else if (b.dtype == DataType::BFLOAT16)      // two bf16 operands
-        check(ttmi_matmul_bf16(a_tiles.data, TTMI_TILE, b.buffer.data, batch_a, batch_b, m, k, n, bias ? bias_row.data : nullptr, activation, c.data,
-                               c_layout, packed_out ? (int)out_dtype : TTMI_BFLOAT16, nullptr, 0, stream_of(device)));
-    else if (a_in_kernel)
+    const void *row = bias ? bias_row.data : nullptr;
+    if (rc != TTMI_ERR_UNSUPPORTED) {
+        check(rc);
+    } else if (b.dtype == DataType::BFLOAT16) {      // two bf16 operands
+        check(ttmi_matmul_bf16(a_tiles.data, TTMI_TILE, b.buffer.data, batch_a, batch_b, m, k, n, row, activation, c.data, c_layout, c_dtype, nullptr, 0,
+                               stream_of(device)));
+    } else if (a_in_kernel) {
         check(ttmi_matmul_bfp_ab((const uint32_t *)a_tiles.data, (int)a.dtype, (const uint32_t *)b.buffer.data, (int)b.dtype, batch_a, batch_b, m, k, n,
-                                 bias ? bias_row.data : nullptr, activation, c.data, c_layout, packed_out ? (int)out_dtype : TTMI_BFLOAT16, nullptr, 0,
-                                 stream_of(device)));
-    else
-        check(ttmi_matmul_bfp(a_tiles.data, TTMI_TILE, (const uint32_t *)b.buffer.data, (int)b.dtype, batch_a, batch_b, m, k, n,
-                              bias ? bias_row.data : nullptr, activation, c.data, c_layout, packed_out ? (int)out_dtype : TTMI_BFLOAT16, nullptr, 0,
-                              stream_of(device)));
+                                 row, activation, c.data, c_layout, c_dtype, nullptr, 0, stream_of(device)));
+    } else {
+        check(ttmi_matmul_bfp(a_tiles.data, TTMI_TILE, (const uint32_t *)b.buffer.data, (int)b.dtype, batch_a, batch_b, m, k, n, row, activation, c.data,
+                              c_layout, c_dtype, nullptr, 0, stream_of(device)));
+    }
     Tensor out;
     out.buffer = std::move(c);
     out.shape.assign(a.shape.begin(), a.shape.end() - 1);

@@ -188,6 +188,10 @@ int ttmi_matmul_bfp_ab(const uint32_t *a, int a_fmt, const uint32_t *b, int b_fm
     return matmul_bfp(args, (hipStream_t)stream);
 }
 
+int ttmi_matmul_bias_tiles_supported(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, int b_dtype, int c_dtype) {
+    return (is_bfp(b_dtype) || b_dtype == TTMI_BFLOAT16) && (k & 31) == 0 && (n & 31) == 0 && matmul_takes_bias_tiles(batch, b_batch, m, k, n, b_dtype, is_bfp(c_dtype)) ? 1 : 0;
+}
+
 int ttmi_matmul_bias_tiles(const void *a, int a_dtype, const void *b, int b_dtype, uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k,
                            uint32_t n, const void *bias, int activation, void *c, int c_layout, int c_dtype, void *stream) {
     if (a_dtype != TTMI_BFLOAT16 && a_dtype != TTMI_BFLOAT8_B) return fail(TTMI_ERR_INVALID_ARGUMENT, "matmul: activation dtype must be BFLOAT16 or BFLOAT8_B here, got %d", a_dtype);
