@@ -224,7 +224,8 @@ TTMI_API int ttmi_matmul_bias_tiles_supported(uint32_t batch, uint32_t b_batch, 
 /* ttmi_matmul_bfp, ttmi_matmul_bfp_ab or ttmi_matmul_bf16 (by a_dtype and b_dtype) with a bias that is read where it lies in TILE
  * layout, as ttnn.linear holds it ([.., 32, N] with the values in row 0: ttnn/cpp/ttnn/operations/matmul.hpp:117-140), so that no
  * untilize runs in front of the GEMM.  Bit for bit what those calls give for the row on its own.
- *   a        TILE layout; a_dtype TTMI_BFLOAT16, or TTMI_BFLOAT8_B for shapes that ttmi_matmul_bfp_ab_supported() names
+ *   a        TILE layout; a_dtype TTMI_BFLOAT16.  TTMI_BFLOAT8_B goes through without a bias only, for shapes that ttmi_matmul_bfp_ab_supported()
+ *            names: those are streamed, and ttmi_matmul_bfp_ab takes their bias as a row
  *   b        b_dtype TTMI_BFLOAT8_B | TTMI_BFLOAT4_B | TTMI_BFLOAT16 (the last with bf16 activations only)
  *   bias     NULL or n / 32 bf16 tiles of 2048 bytes, of which row 0 counts
  * The rest as there, without a workspace.  Shapes whose weights are streamed (ttmi_matmul_bias_tiles_supported: 0), and those that are

@@ -842,6 +842,72 @@ def test_bias_in_tiles_is_the_row_on_its_own(oracle, kernel, batch, m, k, n, kno
         assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
 
 
+def _call_bias_tiles(a, a_dtype, words, fmt, batch, b_batch, m, k, n, bias, activation, c, c_layout, c_dtype):
+    return capi.lib().ttmi_matmul_bias_tiles(a.data_ptr(), a_dtype, words.data_ptr(), fmt, batch, b_batch, m, k, n, None if bias is None else bias.data_ptr(), activation,
+                                             c.data_ptr(), c_layout, c_dtype, torch.cuda.current_stream().cuda_stream)
+
+
+def _bias_in_tiles_and_row(n, seed):
+    row = bf16_dev(workloads.f32_to_bf16_bits_rne(workloads.normal_tensor((n,), seed=seed)))
+    rows = torch.full((1, 32, n), float("nan"), dtype=torch.bfloat16, device="cuda")
+    rows[0, 0] = row.reshape(n)
+    return capi.tilize(rows), row
+
+
+@pytest.mark.parametrize("fmt,kernel,batch,b_batch,m,k,n", [
+    (BFP4, "tile", 2, 1, 96, 160, 288), (BFP4, "expanded", 3, 3, 64, 96, 160), (BFP8, "expanded", 2, 2, 32, 1024, 96), (BFP8, None, 5, 5, 160, 512, 2112),
+    (BFP8, None, 1, 1, 1024, 4096, 4096), (capi.BFLOAT16, "bf16 in place", 2, 2, 64, 96, 160), (capi.BFLOAT16, "bf16 in place", 3, 1, 32, 64, 32),
+    (capi.BFLOAT16, "expanded", 3, 1, 96, 64, 544), (capi.BFLOAT16, None, 1, 1, 32, 4544, 256)])
+def test_bias_in_tiles_for_every_kind_of_weights(fmt, kernel, batch, b_batch, m, k, n, knobs):
+    """ttmi_matmul_bias_tiles with block-float and bf16 weights, common to the slices and one for each, by the routes that take the bias in tiles
+    (k ranges cut or not): the bits of the bias in a row, in both layouts and types of C, with every activation; and without a bias."""
+    if kernel:
+        knobs("kernel", kernel)
+    assert kernel or capi.lib().ttmi_matmul_bias_tiles_supported(batch, b_batch, m, k, n, fmt, capi.BFLOAT16) == 1
+    a = capi.tilize(bf16_dev(workloads.activations_bf16(m, k, seed=440, batch=batch)).reshape(batch, m, k))
+    w = torch.from_numpy(workloads.weights_f32(k, n, seed=441, batch=b_batch)).cuda().reshape(b_batch, k, n)
+    words = capi.tilize(w.bfloat16()) if fmt == capi.BFLOAT16 else capi.pack_tensor(fmt, w)
+    tiles, row = _bias_in_tiles_and_row(n, 442)
+    for activation in (capi.ACT_NONE, capi.ACT_RELU, capi.ACT_GELU, capi.ACT_SILU):
+        for layout in (capi.TILE, capi.ROW_MAJOR):
+            for out_dtype, c_dtype in ((torch.bfloat16, capi.BFLOAT16), (torch.float32, capi.FLOAT32)):
+                for bias in (True, False):
+                    more = {"c_layout": layout, "bias": row if bias else None, "activation": activation, "out_dtype": out_dtype}
+                    if fmt == capi.BFLOAT16:
+                        want = capi.matmul_bf16(a, capi.TILE, words, batch, b_batch, m, k, n, **more)
+                    else:
+                        want = capi.matmul_bfp(a, capi.TILE, words, fmt, batch, b_batch, m, k, n, **more)
+                    got = torch.zeros_like(want)
+                    capi.check(_call_bias_tiles(a, capi.BFLOAT16, words, fmt, batch, b_batch, m, k, n, tiles if bias else None, activation, got, layout, c_dtype))
+                    assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+
+
+@pytest.mark.parametrize("a_dtype,fmt,m,k,n", [(capi.BFLOAT16, BFP8, 32, 1024, 4096), (capi.BFLOAT16, BFP4, 32, 4096, 14336), (capi.BFLOAT16, BFP8, 96, 256, 512),
+                                               (capi.BFLOAT16, BFP8, 224, 4096, 1024), (BFP8, BFP8, 32, 1024, 4096), (BFP8, BFP4, 32, 160, 96)])
+def test_streamed_shapes_refuse_a_bias_in_tiles(a_dtype, fmt, m, k, n, test_library):
+    """Shapes whose weights are streamed: refused with a bias in tiles before anything is launched, C stays as it was; without a bias
+    they go through with the bits of the ordinary call, BFLOAT8_B activations included."""
+    assert a_dtype == BFP8 or test_library.ttmi_matmul_bias_tiles_supported(1, 1, m, k, n, fmt, capi.BFLOAT16) == 0
+    dense = bf16_dev(workloads.activations_bf16(m, k, seed=450)).reshape(1, m, k)
+    a = capi.tilize(dense) if a_dtype == capi.BFLOAT16 else capi.pack_tensor(BFP8, dense.float())
+    words = capi.pack_tensor(fmt, torch.from_numpy(workloads.weights_f32(k, n, seed=451)).cuda().reshape(1, k, n))
+    tiles, _ = _bias_in_tiles_and_row(n, 452)
+    c = torch.full((1, m, n), -7.0, dtype=torch.bfloat16, device="cuda")
+    args = (a, a_dtype, words, fmt, 1, 1, m, k, n)
+    unsupported = 3
+    assert _call_bias_tiles(*args, tiles, capi.ACT_SILU, c, capi.TILE, capi.BFLOAT16) == unsupported
+    torch.cuda.synchronize()
+    assert bool((c == -7.0).all())
+    capi.check(_call_bias_tiles(*args, None, capi.ACT_SILU, c, capi.TILE, capi.BFLOAT16))
+    if a_dtype == BFP8:
+        want = torch.empty_like(c)
+        capi.check(capi.lib().ttmi_matmul_bfp_ab(a.data_ptr(), BFP8, words.data_ptr(), fmt, 1, 1, m, k, n, None, capi.ACT_SILU, want.data_ptr(), capi.TILE, capi.BFLOAT16, None, 0,
+                                                 torch.cuda.current_stream().cuda_stream))
+    else:
+        want = capi.matmul_bfp(a, capi.TILE, words, fmt, 1, 1, m, k, n, c_layout=capi.TILE, activation=capi.ACT_SILU)
+    assert torch.equal(c.reshape(-1).view(torch.int16), want.reshape(-1).view(torch.int16))
+
+
 @pytest.mark.parametrize("fmt", [BFP8, BFP4, capi.BFLOAT16])
 @pytest.mark.parametrize("batch,m,k,n", [(8, 384, 64, 96), (2, 32, 96, 544), (5, 33, 64, 288), (3, 300, 1024, 64), (2, 384, 1024, 320)])
 def test_slices_with_common_weights_as_rows_of_the_expanding_gemm(oracle, fmt, batch, m, k, n, knobs):
