@@ -911,8 +911,8 @@ def test_streamed_shapes_refuse_a_bias_in_tiles(a_dtype, fmt, m, k, n, test_libr
 @pytest.mark.parametrize("fmt", [BFP8, BFP4, capi.BFLOAT16])
 @pytest.mark.parametrize("batch,m,k,n", [(8, 384, 64, 96), (2, 32, 96, 544), (5, 33, 64, 288), (3, 300, 1024, 64), (2, 384, 1024, 320)])
 def test_slices_with_common_weights_as_rows_of_the_expanding_gemm(oracle, fmt, batch, m, k, n, knobs):
-    """Slices joined into rows (fewer blocks, row blocks across slices, odd rows, k ranges cut in neither or in both) give the bits
-    that each slice gives on its own where no k range is cut, in every layout and output type that takes the shape."""
+    """Slices with common weights, joined into rows or not (odd rows, k ranges cut in none or, where k = 1024, in the slices together and each
+    alone, at the same places), give the bits that each slice gives on its own, in every layout and output type that takes the shape."""
     knobs("kernel", "expanded")
     a = bf16_dev(workloads.activations_bf16(m, k, seed=430, batch=batch)).reshape(batch, m, k)
     w = workloads.weights_f32(k, n, seed=431)
@@ -931,10 +931,37 @@ def test_slices_with_common_weights_as_rows_of_the_expanding_gemm(oracle, fmt, b
         operand = lambda x: capi.tilize(x) if layout == capi.TILE else x
         got = product(operand(a), layout, batch, **more).reshape(-1)
         want = torch.cat([product(operand(a[i:i + 1]), layout, 1, **more).reshape(-1) for i in range(batch)])
-        if k < 1024:                                         # one k range everywhere
-            assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
-        elif "out_bfp" not in more:                          # sums in another order: 2K 2^-24 sum |a||w| < 1e-2 here, and a rounding to bf16
-            assert torch.allclose(got.float(), want.float(), rtol=2 ** -7, atol=1e-2)
+        assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
+
+
+# blocks of 256 x 256, of the slices and joined: 176 and 136; 234 and 143, row blocks across slices of odd rows; 200 and 125, which would be cut in
+# two, so they are not joined; 24 and 18, cut either way
+@pytest.mark.parametrize("batch,m,k,n,joined", [(11, 384, 1024, 2048, True), (9, 300, 1024, 3232, True), (8, 130, 1024, 6400, False), (6, 320, 1024, 512, False)])
+@pytest.mark.parametrize("fmt", [BFP8, BFP4])
+def test_which_slices_the_expanding_gemm_joins(fmt, batch, m, k, n, joined, knobs, test_library):
+    """Slices become rows of one where that saves blocks and no k range is cut either way, k ranges long enough to be cut among them:
+    what the route says, and the bits of the slices one by one on a workspace that has no room for the sums of k ranges."""
+    knobs("kernel", "expanded")
+    out = (ctypes.c_uint32 * 4)()
+    test_library.ttmi_test_route(batch, 1, m, k, n, fmt, capi.BFLOAT16, out)
+    assert tuple(out)[:3] == ((4, 1, batch * m) if joined else (4, batch, m))
+    a = bf16_dev(workloads.activations_bf16(m, k, seed=435, batch=batch)).reshape(batch, m, k)
+    words = capi.pack_tensor(fmt, torch.from_numpy(workloads.weights_f32(k, n, seed=436)).cuda().reshape(1, k, n))
+    workspace = torch.empty(capi.lib().ttmi_matmul_bfp_workspace_bytes(1, m, k, n, fmt), dtype=torch.uint8, device="cuda")
+    forms = [(capi.ROW_MAJOR, {}), (capi.ROW_MAJOR, {"out_dtype": torch.float32})]
+    if m % 32 == 0:
+        forms += [(capi.TILE, {"c_layout": capi.TILE}), (capi.TILE, {"c_layout": capi.TILE, "out_bfp": fmt})]
+    for layout, more in forms:
+        operand = lambda x: capi.tilize(x) if layout == capi.TILE else x
+        got = capi.matmul_bfp(operand(a), layout, words, fmt, batch, 1, m, k, n, activation=capi.ACT_RELU, **more).reshape(-1)
+        if out[3]:
+            whole = capi.matmul_bfp(operand(a), layout, words, fmt, batch, 1, m, k, n, activation=capi.ACT_RELU, workspace=workspace, **more).reshape(-1)
+            got, cut = whole, got
+            if more.get("out_dtype") == torch.float32:
+                assert not torch.equal(cut, whole)      # the sums of k ranges are added in another order
+        want = torch.cat([capi.matmul_bfp(operand(a[i:i + 1]), layout, words, fmt, 1, 1, m, k, n, activation=capi.ACT_RELU, workspace=workspace, **more).reshape(-1)
+                          for i in range(batch)])
+        assert torch.equal(got.view(torch.uint8), want.view(torch.uint8))
 
 
 @pytest.mark.parametrize("kernel", [None, "expanded"])
@@ -1081,9 +1108,9 @@ def test_k_ranges_of_the_expanding_gemm(oracle, batch, m, k, n, fmt, knobs):
         assert np.array_equal(packed.cpu().numpy().view(np.uint32), host)
 
 
-# slice by slice (the first two); as rows of one GEMM: of bf16 tiles, of 256 x 256 blocks, of such blocks with the last ones in k ranges,
-# rows that are no multiple of a tile among them, so that tiles and blocks begin in one slice and end in the next
-@pytest.mark.parametrize("batch,m,k,n,route", [(8, 384, 1024, 4096, (4, 8, 384, 0)), (5, 333, 512, 2112, (5, 5, 333, 0)), (64, 32, 1024, 4096, (5, 1, 2048, 0)), (5, 150, 512, 2112, (5, 1, 750, 0)),
+# as rows of one GEMM that joins them itself; slice by slice; as rows of one GEMM: of bf16 tiles, of 256 x 256 blocks, of such blocks with the last
+# ones in k ranges, rows that are no multiple of a tile among them, so that tiles and blocks begin in one slice and end in the next
+@pytest.mark.parametrize("batch,m,k,n,route", [(8, 384, 1024, 4096, (4, 1, 3072, 0)), (5, 333, 512, 2112, (5, 5, 333, 0)), (64, 32, 1024, 4096, (5, 1, 2048, 0)), (5, 150, 512, 2112, (5, 1, 750, 0)),
                                                (9, 333, 1024, 4096, (4, 1, 2997, 0)), (13, 333, 1024, 4096, (4, 1, 4329, 1))])
 def test_slices_that_share_their_weights(batch, m, k, n, route, test_library):
     """Slices with common weights, multiplied as the rows of one GEMM where that is better: float64, dense and tiles alike."""

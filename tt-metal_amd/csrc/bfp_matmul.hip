@@ -1437,11 +1437,13 @@ __attribute__((visibility("default"))) int ttmi_test_kernel_choice(uint32_t batc
     return (int)ttmi::choose_kernel(batch, m, k, n, b_fmt, c_dtype == TTMI_BFLOAT8_B || c_dtype == TTMI_BFLOAT4_B);
 }
 // where a call with scratch of the library's own goes: out[0] the kernel (as above, 5 = bf16 tiles), out[1] the slices it sees (1: folded
-// into rows), out[2] the rows of each, out[3] whether the expanding GEMM cuts k ranges
+// into rows, by the route or by the expanding GEMM itself), out[2] the rows of each, out[3] whether the expanding GEMM cuts k ranges
 __attribute__((visibility("default"))) void ttmi_test_route(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, int b_fmt, int c_dtype, uint32_t out[4]) {
     ttmi::MatmulArgs x{};
     x.batch = batch; x.b_batch = b_batch; x.m = m; x.k = k; x.n = n; x.b_fmt = b_fmt;
-    const ttmi::Route r = ttmi::own_scratch_route(x, c_dtype == TTMI_BFLOAT8_B || c_dtype == TTMI_BFLOAT4_B);
+    ttmi::Route r = ttmi::own_scratch_route(x, c_dtype == TTMI_BFLOAT8_B || c_dtype == TTMI_BFLOAT4_B);
+    x.batch = r.batch; x.m = r.m;
+    if (r.kernel == ttmi::Kernel::Expanded && ttmi::rows_of_one_slice(x)) { r.m *= r.batch; r.batch = 1; }
     out[0] = (uint32_t)r.kernel; out[1] = r.batch; out[2] = r.m;
     out[3] = r.kernel == ttmi::Kernel::Expanded && ttmi::matmul_expanded_scratch_bytes(r.batch, b_batch, r.m, k, n) >= ttmi::matmul_expanded_workspace_bytes(b_batch, k, n) + (1u << 18);
 }

@@ -407,7 +407,7 @@ int validate_expanded(const MatmulArgs &x) {
 // fewer blocks and as many rounds: 384 rows a slice pad to 512.  Only where neither way cuts k ranges, so that the scratch and
 // every sum are what they were.  8 x [384, 1024] x [1024, 4096], BFLOAT8_B weights, 192 blocks against 256 in one round:
 // 34.5 us against 42.8; with GELU and a block-float output 45.7 against 52.3.
-static bool rows_of_one_slice(const MatmulArgs &x) {
+bool rows_of_one_slice(const MatmulArgs &x) {
     const uint64_t rows = (uint64_t)x.batch * x.m;
     if (x.b_batch != 1 || x.batch == 1 || (rows + 31) / 32 * 64 * x.k > 0xffffffffull) return false;       // (validate_expanded: A of 4 GiB)
     const ExpandedPlan slices = plan_expanded(x.batch, 1, x.m, x.k, x.n, 0, true), joined = plan_expanded(1, 1, (uint32_t)rows, x.k, x.n, 0, true);

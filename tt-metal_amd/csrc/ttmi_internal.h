@@ -107,6 +107,7 @@ int matmul_bf16_direct(const MatmulArgs &args, hipStream_t st);    // bf16 weigh
 uint32_t bf16_direct_block(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n);    // the block edge a shape gets there, 0: not for it
 double matmul_direct_estimate(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, double bytes_per_weight);    // us, behind a pass that expands the weights
 int validate_expanded(const MatmulArgs &args);
+bool rows_of_one_slice(const MatmulArgs &args);      // matmul_bfp_expanded runs the slices as the rows of one
 double matmul_expanded_estimate(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n, double bytes_per_weight);   // us, k ranges cut where that helps
 size_t matmul_expanded_workspace_bytes(uint32_t b_batch, uint32_t k, uint32_t n);
 size_t matmul_expanded_scratch_bytes(uint32_t batch, uint32_t b_batch, uint32_t m, uint32_t k, uint32_t n);      // with the partial sums of k ranges
