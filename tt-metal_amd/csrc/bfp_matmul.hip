@@ -1314,8 +1314,8 @@ int matmul_bfp(const MatmulArgs &asked, hipStream_t st) {
     if (a8 && !matmul_takes_bfp_activations(x.batch, x.m, x.k, x.n, x.b_fmt))
         return fail(TTMI_ERR_UNSUPPORTED, "matmul: block-float activations are taken by the one-band streaming kernel only, which this shape does "
                     "not go to (ttmi_matmul_bfp_ab_supported): expand them with ttmi_typecast_tiles first");
-    // The streaming kernels take a bias as a row only: with the index of a tile in their epilogues [96, 4544] x [4544, 4672], which has no
-    // bias at all, took 17.7 us instead of 16.1.
+    // The streaming kernels take a bias as a row only: with the index of a tile selected per column in their epilogues [96, 4544] x [4544, 4672],
+    // which has no bias at all, took 17.7 us instead of 16.1.  Callers ask matmul_takes_bias_tiles first; what gets here found no scratch.
     if (x.bias_tiled && x.bias && (kernel == Kernel::Wide || kernel == Kernel::Stream))
         return fail(TTMI_ERR_UNSUPPORTED, "matmul: the streaming kernels take no bias in tiles: untilize its first row first");
     switch (kernel) {

@@ -406,7 +406,7 @@ int validate_expanded(const MatmulArgs &x) {
 // Slices with common weights run as the rows of one slice (the same memory: dense rows, or whole bands of tiles) where that takes
 // fewer blocks and as many rounds: 384 rows a slice pad to 512.  Only where neither way cuts k ranges, so that the scratch and
 // every sum are what they were.  8 x [384, 1024] x [1024, 4096], BFLOAT8_B weights, 192 blocks against 256 in one round:
-// 34.5 us against 42.8; with GELU and a block-float output 45.7 against 52.3.
+// 34.5 us against 41.2; with GELU and a block-float output 45.5 against 52.3.
 bool rows_of_one_slice(const MatmulArgs &x) {
     const uint64_t rows = (uint64_t)x.batch * x.m;
     if (x.b_batch != 1 || x.batch == 1 || (rows + 31) / 32 * 64 * x.k > 0xffffffffull) return false;       // (validate_expanded: A of 4 GiB)
